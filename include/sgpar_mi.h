@@ -105,9 +105,10 @@ int mi_ctx_set_graphs(mi_ctx* ctx, int enable);
    whatever the level's size.  mixed == 0 (the default): FP64 throughout, as
    the reference.  No counterpart in the reference. */
 int mi_ctx_set_precision(mi_ctx* ctx, int mixed, uint32_t min_entries);
-/* Levels of at most 16384 vertices and at most max_entries stored entries
-   (default 131072; 0: none) run their whole FP64 power iteration in one
-   1024-thread workgroup, chunk iterations per launch at most (0: 8192),
+/* Levels of at most 7168 vertices and at most max_entries stored entries
+   (default 131072, at most 262144; 0: none) run their whole FP64 power
+   iteration in one workgroup, consecutive such levels in one launch, chunk
+   iterations per launch at most (0: 8192),
    instead of two kernel launches per iteration.  Same stop rule and
    result bookkeeping; the sums are added in another order.  No counterpart
    in the reference. */

@@ -248,7 +248,7 @@ class Context:
         self.check(self._L.mi_ctx_set_builder(self.h, builder), "mi_ctx_set_builder")
 
     def set_small_levels(self, max_entries: int = 1 << 17, chunk: int = 0) -> None:
-        """Levels of <= 16384 vertices and <= max_entries entries iterate in one
+        """Levels of <= 7168 vertices and <= max_entries entries iterate in one
         workgroup (0: never), at most chunk iterations per launch (0: 8192)."""
         self.check(self._L.mi_ctx_set_small_levels(self.h, max_entries, chunk), "mi_ctx_set_small_levels")
 

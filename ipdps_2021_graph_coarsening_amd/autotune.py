@@ -2,7 +2,7 @@
 
 Two policies decide how each level of a hierarchy runs its power iteration:
 - which levels iterate inside one workgroup (`mi_ctx_set_small_levels`: at
-  most 16384 vertices and at most `small_max_entries` stored entries), and
+  most 7168 vertices and at most `small_max_entries` stored entries), and
 - which levels above the finest run in mixed precision
   (`mi_ctx_set_precision`: at least `mixed_min_entries` entries).
 

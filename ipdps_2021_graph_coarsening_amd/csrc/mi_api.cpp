@@ -339,6 +339,16 @@ DBuf<double> start_vector(Ctx& c, uint32_t gn, uint64_t* pcg_state, uint64_t pcg
     return cur;
 }
 
+void log_eigenvalue(Ctx& c, const DGraph& g, const double* ev, mi_stats* st)
+{
+    double elog[3];
+    eigen_log_level(c, g, ev, elog);
+    st->has_eigen_log = 1;
+    st->eigenvalue = elog[0];
+    st->eigen_min = elog[1];
+    st->eigen_max = elog[2];
+}
+
 // The levels `from` .. 0 of the eigensolve, cur holding the start vector of
 // level `from`; returns the finest-level eigenvector.
 DBuf<double> fiedler_levels(Ctx& c, const std::vector<DLevel>& lv, int from, DBuf<double> cur, int normLap,
@@ -368,15 +378,51 @@ DBuf<double> fiedler_levels(Ctx& c, const std::vector<DLevel>& lv, int from, DBu
             level_keys(c, key[l].get(), lv[l].vcmap.get(), lv[l].g.n, key[l + 1].get(), lv[l + 1].g.n);
         }
     }
+    auto mixed_at = [&](int l) { return c.mixed && l > 0 && lv[l].g.m >= c.mixed_min_m; };
     for (int l = from; l >= 0; l--) {
         PowerStats ps;
+        // consecutive small levels: one launch
+        int e = l;
+        while (e >= 0 && !local[e] && small_level(c, lv[e].g, mixed_at(e))) e--;
+        if (e < l) {
+            const int last = e + 1;
+            std::vector<SmallChain> chain(1);
+            for (int k = l; k >= last; k--) {
+                SmallChainLevel s;
+                s.g = &lv[k].g;
+                s.vcmap = k == l ? nullptr : lv[k].vcmap.get();
+                chain[0].lv.push_back(s);
+            }
+            DBuf<double> res(&c.pool, lv[last].g.n);
+            chain[0].start = cur.get();
+            chain[0].out = res.get();
+            solve_small_chains(c, chain, normLap, tol);
+            cur = std::move(res);
+            if (st) {
+                for (int k = l; k >= last && k < MI_MAX_LEVELS; k--) {
+                    const SmallChainLevel& s = chain[0].lv[l - k];
+                    st->level_iters[k] = s.iters;
+                    st->level_max_reached[k] = s.max_reached;
+                    st->level_eigen_ms[k] = s.ms;
+                }
+                if (last == 0 && !normLap) log_eigenvalue(c, lv[0].g, cur.get(), st);
+            }
+            l = last;
+            if (l > 0) {
+                const uint32_t nf = lv[l - 1].g.n;
+                DBuf<double> fine(&c.pool, nf);
+                prolong(c, lv[l - 1].vcmap.get(), nf, cur.get(), fine.get());
+                cur = std::move(fine);
+            }
+            continue;
+        }
         // the reference logs the eigenvalue after the final (finest) solve
         // with the Laplacian (eigensolve_kokkos.h:201-203)
         double elog[3];
         const bool log_here = st && l == 0 && !normLap;
         // mixed precision: FP32 iterations on the large levels above the
         // finest, whose FP64 solve is the final refinement
-        const bool mixed = c.mixed && l > 0 && lv[l].g.m >= c.mixed_min_m;
+        const bool mixed = mixed_at(l);
         if (st && mixed) st->mixed++;
         if (local[l]) {
             DGraph pg;
@@ -1036,50 +1082,46 @@ void bisect_many(Ctx& c, const std::vector<const DGraph*>& gs, const mi_config* 
     // k is batched when every coarser level is
     std::vector<DBuf<double>> cur(K);
     std::vector<int> lo(K);
-    int depth = 0;
+    std::vector<DBuf<double>> out(K);
+    std::vector<SmallChain> chains;
+    std::vector<size_t> who;
     for (size_t k = 0; k < K; k++) {
         const int L = (int)H[k].size();
         MI_CHECK(L >= 1, ST_STATE, "empty hierarchy");
         cur[k] = start_vector(c, H[k][L - 1].g.n, chain ? &pcg_states[0] : &pcg_states[k], pcg_inc);
-        int l = L - 1;
-        while (l >= 0) {
-            const DGraph& g = H[k][l].g;
-            const bool mixed = c.mixed && l > 0 && g.m >= c.mixed_min_m;
-            if (!small_lds_level(c, g, mixed)) break;
-            l--;
-        }
-        lo[k] = l + 1;
-        depth = std::max(depth, L - lo[k]);
         if (stats) {
             stats[k].has_eigen_log = 0;
             stats[k].mixed = 0;
         }
-    }
-    std::vector<std::vector<DBuf<double>>> out(K);
-    for (size_t k = 0; k < K; k++) out[k].resize(H[k].size());
-    for (int d = 0; d < depth; d++) {
-        std::vector<BatchLevel> jobs;
-        std::vector<std::pair<size_t, int>> who;
-        for (size_t k = 0; k < K; k++) {
-            const int L = (int)H[k].size(), l = L - 1 - d;
-            if (l < lo[k]) continue;
-            BatchLevel b;
-            b.g = &H[k][l].g;
-            b.start = d == 0 ? cur[k].get() : out[k][l + 1].get();
-            b.vcmap = d == 0 ? nullptr : H[k][l].vcmap.get();
-            out[k][l] = DBuf<double>(&c.pool, H[k][l].g.n);
-            b.out = out[k][l].get();
-            jobs.push_back(b);
-            who.emplace_back(k, l);
+        SmallChain ch;
+        int l = L - 1;
+        for (; l >= 0; l--) {
+            const DGraph& g = H[k][l].g;
+            const bool mixed = c.mixed && l > 0 && g.m >= c.mixed_min_m;
+            if (!small_level(c, g, mixed)) break;
+            SmallChainLevel s;
+            s.g = &g;
+            s.vcmap = l == L - 1 ? nullptr : H[k][l].vcmap.get();
+            ch.lv.push_back(s);
         }
-        power_iter_small_batch(c, jobs, normLap, tol);
-        for (size_t j = 0; j < jobs.size(); j++) {
-            const size_t k = who[j].first;
-            const int l = who[j].second;
-            if (stats && l < MI_MAX_LEVELS) {
-                stats[k].level_iters[l] = jobs[j].iters;
-                stats[k].level_max_reached[l] = jobs[j].max_reached;
+        lo[k] = l + 1;
+        if (lo[k] == L) continue;
+        out[k] = DBuf<double>(&c.pool, H[k][lo[k]].g.n);
+        ch.start = cur[k].get();
+        ch.out = out[k].get();
+        chains.push_back(std::move(ch));
+        who.push_back(k);
+    }
+    solve_small_chains(c, chains, normLap, tol);
+    for (size_t j = 0; stats && j < chains.size(); j++) {
+        const size_t k = who[j];
+        int l = (int)H[k].size() - 1;
+        for (const SmallChainLevel& s : chains[j].lv) {
+            if (l < MI_MAX_LEVELS) {
+                stats[k].level_iters[l] = s.iters;
+                stats[k].level_max_reached[l] = s.max_reached;
             }
+            l--;
         }
     }
     MI_HIP(hipStreamSynchronize(c.stream));
@@ -1098,20 +1140,13 @@ void bisect_many(Ctx& c, const std::vector<const DGraph*>& gs, const mi_config* 
             ev[k] = fiedler_levels(w, H[k], L - 1, std::move(x), normLap, tol, st);
         } else if (lo[k] == 0) {
             ev[k] = DBuf<double>(&w.pool, H[k][0].g.n);
-            MI_HIP(hipMemcpyAsync(ev[k].get(), out[k][0].get(), (size_t)H[k][0].g.n * 8, hipMemcpyDeviceToDevice,
+            MI_HIP(hipMemcpyAsync(ev[k].get(), out[k].get(), (size_t)H[k][0].g.n * 8, hipMemcpyDeviceToDevice,
                                   w.stream));
-            if (st && !normLap) {
-                double elog[3];
-                eigen_log_level(w, H[k][0].g, ev[k].get(), elog);
-                st->has_eigen_log = 1;
-                st->eigenvalue = elog[0];
-                st->eigen_min = elog[1];
-                st->eigen_max = elog[2];
-            }
+            if (st && !normLap) log_eigenvalue(w, H[k][0].g, ev[k].get(), st);
         } else {
             const int l = lo[k] - 1;
             DBuf<double> fine(&w.pool, H[k][l].g.n);
-            prolong(w, H[k][l].vcmap.get(), H[k][l].g.n, out[k][l + 1].get(), fine.get());
+            prolong(w, H[k][l].vcmap.get(), H[k][l].g.n, out[k].get(), fine.get());
             ev[k] = fiedler_levels(w, H[k], l, std::move(fine), normLap, tol, st);
         }
     });

@@ -187,23 +187,29 @@ struct PowerStats {
 // deflation, sums, normalisation and stopping test stay FP64.
 void power_iter(Ctx& c, const DGraph& g, double* d_u, int normLap, double tol, PowerStats* st,
                 double* eig_log = nullptr, bool mixed = false);
-// A small level (small_lds_level) solved by power_iter_small_batch: its start
-// vector is start[vcmap[i]] (start[i] when vcmap is null), orthogonalised
-// and normalised as power_iter does; its result goes to out (n doubles).
-struct BatchLevel {
+// Consecutive small levels of one hierarchy, coarsest first, solved in one
+// workgroup: the first one's start vector is start (or start[vcmap[i]]),
+// each following one's is the previous result prolonged by its vcmap; each is
+// orthogonalised and normalised as power_iter does, and the last one's
+// result goes to out (which may be start).
+struct SmallChainLevel {
     const DGraph* g = nullptr;
-    const double* start = nullptr;
-    const uint32_t* vcmap = nullptr;
-    double* out = nullptr;
-    uint64_t iters = 0;  // results
+    const uint32_t* vcmap = nullptr;  // vertices of g -> vertices of the vector before (null: the same)
+    uint64_t iters = 0;               // results
     int max_reached = 0;
+    double ms = 0;
 };
-// Whether power_iter runs level g in one workgroup with every vector in LDS
-// (so that it can be batched); mixed: the level would run in mixed precision.
-bool small_lds_level(const Ctx& c, const DGraph& g, bool mixed);
-// The FP64 power iterations of independent small levels in one launch (one
-// workgroup each): the same results, bit for bit, as power_iter on each.
-void power_iter_small_batch(Ctx& c, std::vector<BatchLevel>& lv, int normLap, double tol);
+struct SmallChain {
+    std::vector<SmallChainLevel> lv;
+    const double* start = nullptr;
+    double* out = nullptr;
+};
+// Whether power_iter runs level g in one workgroup (so that it can be chained
+// and batched); mixed: the level would run in mixed precision.
+bool small_level(const Ctx& c, const DGraph& g, bool mixed);
+// The FP64 power iterations of independent chains in one launch, one
+// workgroup each: the same results, bit for bit, as power_iter level by level.
+void solve_small_chains(Ctx& c, std::vector<SmallChain>& chains, int normLap, double tol);
 // The final eigenvalue log (eigenvalue, min, max) of level g for vector d_u.
 void eigen_log_level(Ctx& c, const DGraph& g, const double* d_u, double* out3);
 // Locality order for the solve of a level.  gather_form_level: the level's

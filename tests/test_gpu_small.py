@@ -1,0 +1,126 @@
+"""Small levels' power iteration (one workgroup, csrc/mi_small.hip) at the
+sizes where its layout changes: one wavefront (<= 64 rows), 4 / 8 / 16
+wavefronts, the largest level and the one after it, rows of very different
+lengths (a hub makes a wavefront's stream too long for registers, then for
+LDS), rows without entries, and weights past the packed entry's 19 bits.
+
+Reference: numpy FP64, the reference's formulas (eigensolve_kokkos.h:102-206)
+run for the number of iterations the device reports.  Both start from the
+same vector and each step is a contraction up to rounding, so the vectors
+differ by at most a few eps per iteration: 300 iterations of 1e-15 stay below
+1e-12; 1e-11 is allowed.  With normLap the loop takes the constant vector out
+only once, before the first iteration, and its component, of rounding size in
+both runs, then grows towards the others (its eigenvalue is the largest) and
+rescales the normalised vector: the constant and the vector itself are
+projected out of the difference there.  The iteration count itself is checked by the change
+of u . v at the device's last and last but one iteration against tol."""
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+from ipdps_2021_graph_coarsening_amd import graphs
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-7
+
+
+def _host(rp, col, w, u, normLap, iters):
+    n = len(rp) - 1
+    A = sp.csr_matrix((np.ones(len(col)) if w is None else w.astype(np.float64), col, rp), shape=(n, n))
+    deg = np.asarray(A.sum(axis=1)).ravel()
+    c = 1 / np.sqrt(n)
+    u = u - (u @ np.full(n, c)) * c if not normLap else u - (u * deg).sum() * c / (c * c * deg.sum()) * c
+    v = u / np.linalg.norm(u)
+    gb = max(2 * deg.max(), 2)
+    dots = [1.0, 0.0]
+    for _ in range(iters):
+        u = v
+        if normLap:
+            v = 0.5 * u + 0.5 * (A @ u) / deg
+        else:
+            v = (gb - deg) * u + A @ u
+            v = v - (v.sum() * c) * c
+        v = v / np.linalg.norm(v)
+        dots.append(u @ v)
+    return u, dots
+
+
+def _star(n, extra, rng):
+    """A hub joined to every vertex, plus random edges."""
+    i = np.arange(1, n)
+    u = np.concatenate([np.zeros(n - 1, np.int64), rng.integers(0, n, extra)])
+    v = np.concatenate([i, rng.integers(0, n, extra)])
+    return graphs.from_edges(n, u, v, None, lcc=False)
+
+
+def _sparse(n, m, rng, wmax):
+    u, v = rng.integers(0, n, m), rng.integers(0, n, m)
+    k = np.arange(n - 1)
+    return graphs.from_edges(n, np.concatenate([u, k]), np.concatenate([v, k + 1]),
+                             rng.integers(1, wmax + 1, m + n - 1), lcc=False)
+
+
+def _case(name):
+    rng = np.random.default_rng(7)
+    kind, n = name.rsplit("-", 1)
+    n = int(n)
+    if kind == "path":
+        return graphs.path(n)
+    if kind == "star":
+        return _star(n, 3 * n, rng)
+    if kind == "dense":
+        return _sparse(n, 20 * n, rng, 9)
+    if kind == "wide":
+        return _sparse(n, 3 * n, rng, 1 << 24)
+    if kind == "w17":
+        return _sparse(n, 3 * n, rng, 1 << 17)
+    return _sparse(n, 2 * n, rng, 16)
+
+
+@pytest.mark.parametrize("name", [
+    "path-2", "path-3", "mesh-17", "star-40", "mesh-63", "mesh-64", "mesh-65", "star-64", "wide-50", "wide-300",
+    "mesh-128", "mesh-129", "mesh-1023", "mesh-1024", "mesh-1025", "star-1000", "star-3000", "dense-900",
+    "dense-2100", "w17-700", "w17-1500", "wide-1500", "wide-6000", "mesh-4096", "mesh-6500", "mesh-7168", "mesh-7169",
+    "star-7168", "dense-4000"])
+@pytest.mark.parametrize("normLap", [0, 1])
+def test_small_level_against_numpy(ctx, name, normLap):
+    rp, col, w = _case(name)
+    n = len(rp) - 1
+    u0 = np.random.default_rng(n).uniform(-1, 1, n)
+    g = ctx.graph(rp, col, w)
+    u, it, mr = g.power_iter(u0, normLap=normLap, tol=TOL)
+    try:
+        ctx.set_small_levels(1 << 17, 3)  # three iterations per launch
+        u3, it3, _ = g.power_iter(u0, normLap=normLap, tol=TOL)
+    finally:
+        ctx.set_small_levels()
+    g.close()
+    assert it3 == it and np.array_equal(u3, u)
+    assert not mr
+    hu, dots = _host(rp, col, w, u0, normLap, it)
+    if n > 2:
+        d = u - hu
+        if normLap:
+            span = np.stack([np.ones(n), hu], axis=1)
+            d = d - span @ np.linalg.lstsq(span, d, rcond=None)[0]
+        assert np.linalg.norm(d) <= 1e-11 * np.linalg.norm(hu)
+    if n > 2 and not normLap:
+        assert abs(dots[-1] - dots[-2]) <= TOL * (1 + 1e-6) or np.isnan(dots[-1])
+        assert it == 1 or abs(dots[-2] - dots[-3]) > TOL * (1 - 1e-6)
+
+
+def test_rows_without_entries(ctx):
+    """Isolated vertices (their rows come last in the layout, in slices of no
+    steps): y = (gb - 0) x there."""
+    rng = np.random.default_rng(3)
+    for n, k in ((60, 20), (700, 300), (5000, 4000)):
+        rp, col, w = _sparse(k, 3 * k, rng, 5)
+        rp = np.concatenate([rp, np.full(n - k, rp[-1], np.uint32)])
+        u0 = rng.uniform(-1, 1, n)
+        g = ctx.graph(rp, col, w)
+        u, it, _ = g.power_iter(u0, tol=TOL)
+        g.close()
+        hu, dots = _host(rp, col, w, u0, 0, it)
+        assert np.linalg.norm(u - hu) <= 1e-11 * np.linalg.norm(hu)
+        assert abs(dots[-1] - dots[-2]) <= TOL * (1 + 1e-6)
