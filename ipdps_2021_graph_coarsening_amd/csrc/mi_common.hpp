@@ -137,7 +137,8 @@ enum Counter : int {
     CT_DONE = 2,     // power iteration finished flag
     CT_MAXR = 3,     // iteration cap reached
     CT_ERR = 4,      // a kernel found a violated size invariant
-    CT_ITER = 5,     // power iteration: launches whose finish kernel has run
+    CT_ITER = 5,     // power iteration: launches whose sums are written
+    CT_ITER2 = 6,    // ... the second counter of the one-launch form, whose launches read one and write the other
     CT_COUNT = 16
 };
 
@@ -209,6 +210,30 @@ __device__ __forceinline__ double wave_sum(double v)
     const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, WAVE - 1);
     const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), WAVE - 1);
     return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+__device__ __forceinline__ uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+
+constexpr int NXCD = 8;
+
+// XCD-aware renumbering of workgroups: workgroup b runs on XCD b % 8; the
+// logical indices of one XCD are consecutive, so each XCD streams one
+// contiguous part of the matrix.
+__device__ __forceinline__ uint32_t logical_block()
+{
+    const uint32_t nb = gridDim.x, b = blockIdx.x;
+    const uint32_t xq = b % NXCD, q = nb / NXCD, rem = nb % NXCD;
+    return xq * q + (xq < rem ? xq : rem) + b / NXCD;
+}
+
+// Orders this wavefront's LDS accesses before and after it for every lane
+// (LDS operations of one wavefront execute in order: the compiler must keep
+// them so, too).
+__device__ __forceinline__ void wave_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 __device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v)

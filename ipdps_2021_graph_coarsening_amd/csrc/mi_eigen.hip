@@ -46,7 +46,8 @@
 // y, and the four sums, reduced per workgroup.  Every sum has a fixed order,
 // so results are bit-identical run to run.
 //
-// Small levels run the whole loop in one workgroup (mi_small.hip).  Value
+// Small levels run the whole loop in one workgroup (mi_small.hip), levels
+// without long rows one launch per iteration (mi_rows.hip).  Value
 // type V = float is the mixed-precision form of the two kernels above.
 #include "mi_kernels.hpp"
 
@@ -65,7 +66,6 @@ constexpr int SEG = 8;                  // consecutive entries per lane and pass
 constexpr uint32_t PASS = WAVE * SEG;   // entries per wavefront pass
 constexpr uint32_t RINF = 0xFFFFFFFFu;  // row id of the lanes past the last entry
 constexpr uint32_t HEADF = 0x80000000u; // range metadata: the first row began earlier
-constexpr int NXCD = 8;
 constexpr int NW = BLOCK / WAVE;        // wavefronts per workgroup, global-gather form
 constexpr int LBLOCK = 1024;            // workgroup of the LDS form
 constexpr int LNW = LBLOCK / WAVE;      // its wavefronts
@@ -85,16 +85,6 @@ constexpr int NSUM = 5;                 // sums per finish workgroup (the fifth 
 constexpr int W_UNIT = 0, W_U16 = 1, W_U32 = 2;  // weight formats of the streamed arrays
 
 inline unsigned grid1(uint64_t n) { return (unsigned)ceil_div(n ? n : 1, BLOCK); }
-
-// XCD-aware renumbering of workgroups: workgroup b runs on XCD b % 8; the
-// logical indices of one XCD are consecutive, so each XCD streams one
-// contiguous part of the matrix.
-__device__ __forceinline__ uint32_t logical_block()
-{
-    const uint32_t nb = gridDim.x, b = blockIdx.x;
-    const uint32_t xq = b % NXCD, q = nb / NXCD, rem = nb % NXCD;
-    return xq * q + (xq < rem ? xq : rem) + b / NXCD;
-}
 
 // Block layout of a level: block q holds entries [boff[q], boff[q+1]) and its
 // ranges start at range index bwave[q].
@@ -1347,34 +1337,32 @@ __global__ void k_materialize(uint32_t n, const V* __restrict__ y, double* __res
     if (i < n) u[i] = ((double)y[i] - scal[SC_A]) * scal[SC_S];
 }
 
-__global__ void k_to_f32(uint32_t n, const double* __restrict__ x, float* __restrict__ y)
-{
-    uint32_t i = blockIdx.x * BLOCK + threadIdx.x;
-    if (i < n) y[i] = (float)x[i];
-}
-
 // weighted degrees as u32 sums (wrapping like the reference's sgp_wgt_t),
-// one wavefront per row: exact whatever the vector precision
-// one wavefront per row; a row of more than WDEG_LONG entries is listed
+// exact whatever the vector precision
+// LANES lanes per row; a row of more than WDEG_LONG entries is listed
 // (order free: integer sums) for k_wdeg_long instead, so no wavefront walks
 // a hub row alone
 constexpr uint32_t WDEG_LONG = 2048;
+template <int LANES>
 __global__ void __launch_bounds__(BLOCK) k_wdeg_int(uint32_t n, const uint32_t* __restrict__ rowptr,
                                                     const uint32_t* __restrict__ w, uint32_t* __restrict__ wdeg,
                                                     uint32_t* __restrict__ longs, uint32_t* __restrict__ nlong)
 {
-    const uint32_t r = blockIdx.x * NW + threadIdx.x / WAVE;
-    if (r >= n) return;
-    const uint32_t lane = threadIdx.x & (WAVE - 1);
+    const uint64_t i = ((uint64_t)blockIdx.x * BLOCK + threadIdx.x) / LANES;
+    const uint32_t r = i < n ? (uint32_t)i : n - 1, lane = threadIdx.x % LANES;  // (idle lanes: with the last row)
     const uint32_t e0 = rowptr[r], e1 = rowptr[r + 1];
-    if (e1 - e0 > WDEG_LONG) {
-        if (lane == 0) longs[atomicAdd(nlong, 1u)] = r;
-        return;
-    }
+    const bool is_long = e1 - e0 > WDEG_LONG;
     uint32_t t = 0;
-    for (uint32_t e = e0 + lane; e < e1; e += WAVE) t += w[e];
-    t = wave_sum_u32(t);
-    if (lane == 0) wdeg[r] = t;
+    if (!is_long)
+        for (uint32_t e = e0 + lane; e < e1; e += LANES) t += w[e];
+#pragma unroll
+    for (int o = LANES / 2; o > 0; o >>= 1) t += __shfl_xor(t, o, WAVE);
+    if (i < n && lane == 0) {
+        if (is_long)
+            longs[atomicAdd(nlong, 1u)] = r;
+        else
+            wdeg[r] = t;
+    }
 }
 
 // the listed long rows, one workgroup each in turn (fixed grid)
@@ -1825,9 +1813,33 @@ void launch_finish(Ctx& c, int normLap, const StepArgs& A)
         launch_finish_t<false>(c, normLap, A);
 }
 
-// One step = the streaming kernel then the finish kernel.
-void launch_step(Ctx& c, int normLap, const StepArgs& A)
+// A step of a level: by rows (one kernel), or the streaming kernel then the
+// finish kernel.
+struct LevelStep {
+    bool by_rows;
+    bool f32;
+    RowStep rows;
+    StepArgs stream;
+};
+
+LevelStep level_step(Ctx& c, const DGraph& g, const LevelPlan& p, const uint32_t* wdeg, const uint32_t* gb,
+                     const void* yprev, void* ynew, double tol, int mode, int parity)
 {
+    LevelStep L{p.rows.on, p.f32, {}, {}};
+    if (L.by_rows)
+        L.rows = rows_step(c, g, p.rows, wdeg, gb, yprev, ynew, tol, mode, parity);
+    else
+        L.stream = make_args(c, g, p, wdeg, gb, yprev, ynew, tol, mode);
+    return L;
+}
+
+void launch_step(Ctx& c, int normLap, const LevelStep& L)
+{
+    if (L.by_rows) {
+        launch_rows(c, normLap, L.f32, L.rows);
+        return;
+    }
+    const StepArgs& A = L.stream;
     launch_stream(c, A);
     if (A.dense) {
         const unsigned g = (unsigned)ceil_div(A.nwaves ? A.nwaves : 1u, BLOCK);
@@ -1866,6 +1878,13 @@ void plan_level(Ctx& c, const DGraph& g, LevelPlan& p, bool f32)
     const uint32_t n = g.n, m = g.m;
     MI_CHECK(n > 0, ST_ARG, "empty level");
     const uint32_t ncb = column_blocks(n, m);
+    // One launch per iteration where no row is long and x would not be split
+    // into column blocks: the streaming form's second launch and row ids cost
+    // more than gathers from the caches instead of LDS (us per iteration,
+    // before and now: 3d grid 128^3, 2.1 M vertices 73 and 47; its levels of
+    // 628,115 44 and 35, of 183,554 20.5 and 18, of 48,419 15.0 and 12.5, of
+    // 11,686, whose x fits in LDS whole, 15.6 and 9.7).
+    if (ncb <= 1 && plan_rows(c, g, p.rows)) return;
     p.ncb = ncb;
     p.bw = ncb ? (uint32_t)ceil_div(n, ncb) : 0u;
     for (int q = 0; q <= MAXCB; q++) p.boff[q] = p.bwave[q] = 0;
@@ -2127,8 +2146,14 @@ void weighted_degree(Ctx& c, const DGraph& g, const LevelPlan& p, uint32_t* wdeg
         } else {
             DBuf<uint32_t> longs(&c.pool, g.n), nlong(&c.pool, 1);
             fill_u32(c, nlong.get(), 1, 0u);
-            k_wdeg_int<<<(unsigned)ceil_div(g.n, NW), BLOCK, 0, c.stream>>>(g.n, g.R(), g.W(), wdeg, longs.get(),
-                                                                            nlong.get());
+            // lanes per row by the mean row length, so that short rows do
+            // not leave most of a wavefront idle
+            if ((uint64_t)g.m < 16ull * g.n)
+                k_wdeg_int<8><<<(unsigned)ceil_div(8ull * g.n, BLOCK), BLOCK, 0, c.stream>>>(
+                    g.n, g.R(), g.W(), wdeg, longs.get(), nlong.get());
+            else
+                k_wdeg_int<WAVE><<<(unsigned)ceil_div(g.n, NW), BLOCK, 0, c.stream>>>(g.n, g.R(), g.W(), wdeg,
+                                                                                     longs.get(), nlong.get());
             MI_HIP(hipGetLastError());
             const uint32_t ncu = c.num_cu > 0 ? (uint32_t)c.num_cu : 256u;
             k_wdeg_long<<<4 * ncu, BLOCK, 0, c.stream>>>(g.R(), g.W(), wdeg, longs.get(), nlong.get());
@@ -2146,27 +2171,31 @@ void weighted_degree(Ctx& c, const DGraph& g, const LevelPlan& p, uint32_t* wdeg
 void spmv_shift(Ctx& c, const DGraph& g, const LevelPlan& p, const uint32_t* wdeg, const uint32_t* gb_dev,
                 const double* x, double* y)
 {
-    StepArgs A = make_args(c, g, p, wdeg, gb_dev, x, y, 0.0, 1);
-    launch_step(c, 0, A);
+    DBuf<double> xp;
+    if (p.rows.on) {
+        xp = DBuf<double>(&c.pool, (uint64_t)g.n + 1);
+        pad_copy(c, g.n, x, xp.get());
+        x = xp.get();
+    }
+    launch_step(c, 0, level_step(c, g, p, wdeg, gb_dev, x, y, 0.0, 1, 0));
 }
 
 void bench_power_step(Ctx& c, const DGraph& g, int reps, StepBench* out)
 {
     const uint32_t n = g.n;
     DBuf<uint32_t> wdeg(&c.pool, n), gb(&c.pool, 1);
-    DBuf<double> x(&c.pool, n), y(&c.pool, n);  // (float vectors use their first halves)
+    DBuf<double> x(&c.pool, (uint64_t)n + 1), y(&c.pool, (uint64_t)n + 1);  // (float vectors use their first halves)
     LevelPlan p;
     plan_level(c, g, p, c.mixed);  // the precision the context runs in
     weighted_degree(c, g, p, wdeg.get(), gb.get());
     std::vector<double> h(n);
     for (uint32_t i = 0; i < n; i++) h[i] = 1.0 / (1.0 + (i % 97));
-    MI_HIP(hipMemcpyAsync(x.get(), h.data(), (size_t)n * 8, hipMemcpyHostToDevice, c.stream));
-    if (c.mixed) {
-        k_to_f32<<<grid1(n), BLOCK, 0, c.stream>>>(n, x.get(), reinterpret_cast<float*>(y.get()));
-        MI_HIP(hipGetLastError());
-        MI_HIP(hipMemcpyAsync(x.get(), y.get(), (size_t)n * 4, hipMemcpyDeviceToDevice, c.stream));
-    }
-    StepArgs A = make_args(c, g, p, wdeg.get(), gb.get(), x.get(), y.get(), 0.0, 1);
+    MI_HIP(hipMemcpyAsync(y.get(), h.data(), (size_t)n * 8, hipMemcpyHostToDevice, c.stream));
+    if (c.mixed)
+        pad_copy(c, n, y.get(), reinterpret_cast<float*>(x.get()));
+    else
+        pad_copy(c, n, y.get(), x.get());
+    const LevelStep A = level_step(c, g, p, wdeg.get(), gb.get(), x.get(), y.get(), 0.0, 1, 0);
     launch_step(c, 0, A);  // warm-up
     MI_HIP(hipStreamSynchronize(c.stream));
     hipEvent_t e0, e1, e2;
@@ -2177,7 +2206,12 @@ void bench_power_step(Ctx& c, const DGraph& g, int reps, StepBench* out)
     MI_HIP(hipEventRecord(e0, c.stream));
     for (int r = 0; r < reps; r++) launch_step(c, 0, A);
     MI_HIP(hipEventRecord(e1, c.stream));
-    for (int r = 0; r < reps; r++) launch_stream(c, A);
+    for (int r = 0; r < reps; r++) {
+        if (A.by_rows)
+            launch_step(c, 0, A);  // (its one kernel)
+        else
+            launch_stream(c, A.stream);
+    }
     MI_HIP(hipEventRecord(e2, c.stream));
     MI_HIP(hipEventSynchronize(e2));
     float ms_step = 0, ms_stream = 0;
@@ -2199,6 +2233,8 @@ void bench_power_step(Ctx& c, const DGraph& g, int reps, StepBench* out)
     const double wb = g.unit ? 0.0 : (p.w16.get() ? 2.0 : 4.0);
     const double vb = p.f32 ? 4.0 : 8.0;
     out->impl_bytes = (colb + ridb + wb) * g.m + vb * n + vb * (p.ncb > 1 ? p.ncb : 1) * n;
+    if (p.rows.on)  // (padding included; no row ids but one word per row, the vector read and written)
+        out->impl_bytes = (4.0 + (g.unit ? 0.0 : p.rows.w16 ? 2.0 : 4.0)) * (double)p.rows.slots + (2 * vb + 8.0) * n;
     if (p.f32) {  // x and the row partials in FP32
         out->stream_bytes -= 4.0 * n;
         out->step_bytes -= 12.0 * n;
@@ -2292,7 +2328,7 @@ static void eigenvalue_log(Ctx& c, const DGraph& g, const double* d_u, const dou
 }
 
 // The iteration loop of a level as launches of the two-kernel step.
-static void run_steps(Ctx& c, int normLap, const StepArgs (&A)[2])
+static void run_steps(Ctx& c, int normLap, const LevelStep (&A)[2], unsigned long long iter_max)
 {
     // Every launch of this level has the same arguments but for the ping-pong
     // parity (the iteration index lives on the device), so a chunk of
@@ -2344,7 +2380,7 @@ static void run_steps(Ctx& c, int normLap, const StepArgs (&A)[2])
     hipEvent_t* ev = evs.e;
     MI_HIP(hipEventCreateWithFlags(&ev[0], hipEventDisableTiming));
     MI_HIP(hipEventCreateWithFlags(&ev[1], hipEventDisableTiming));
-    const unsigned long long cap = A[0].iter_max + 4ull * GRAPH_ITERS;  // the device stops at iter_max
+    const unsigned long long cap = iter_max + 4ull * GRAPH_ITERS;  // the device stops at iter_max
     // eager launches start with chunks of 2 (a level that stops after a few
     // iterations queues few no-op launches) and double up to GRAPH_ITERS
     uint32_t chunk = graph.x ? GRAPH_ITERS : 2u;
@@ -2389,8 +2425,8 @@ void power_iter(Ctx& c, const DGraph& g, double* d_u, int normLap, double tol, P
         return;
     }
     DBuf<uint32_t> wdeg(&c.pool, n), gb(&c.pool, 1);
-    DBuf<double> other(&c.pool, n);
-    DBuf<float> f0, f1;  // the mixed form's FP32 vectors
+    DBuf<double> d0, d1;  // the loop's vectors
+    DBuf<float> f0, f1;   // ... in the mixed form
     LevelPlan plan;
     plan_level(c, g, plan, mixed);
     weighted_degree(c, g, plan, wdeg.get(), gb.get());
@@ -2414,34 +2450,54 @@ void power_iter(Ctx& c, const DGraph& g, double* d_u, int normLap, double tol, P
     // Launch i (1-based) reads y_{i-1} from buf[(i-1) & 1] and writes y_i to
     // the other buffer; its streaming kernel first decides whether iteration
     // i-1 was the last, so the loop ends one launch after the last iteration.
-    void* buf[2] = {d_u, other.get()};
+    void* buf[2];
     if (mixed) {
         // FP32 vectors from the FP64 start vector (set up in FP64 above)
-        f0 = DBuf<float>(&c.pool, n);
-        f1 = DBuf<float>(&c.pool, n);
-        k_to_f32<<<grid1(n), BLOCK, 0, c.stream>>>(n, d_u, f0.get());
-        MI_HIP(hipGetLastError());
+        f0 = DBuf<float>(&c.pool, (uint64_t)n + 1);
+        f1 = DBuf<float>(&c.pool, (uint64_t)n + 1);
+        pad_copy(c, n, d_u, f0.get());
         buf[0] = f0.get();
         buf[1] = f1.get();
+    } else {
+        d1 = DBuf<double>(&c.pool, (uint64_t)n + 1);
+        buf[0] = d_u;
+        buf[1] = d1.get();
+        if (plan.rows.on) {
+            d0 = DBuf<double>(&c.pool, (uint64_t)n + 1);
+            pad_copy(c, n, d_u, d0.get());
+            buf[0] = d0.get();
+        }
     }
+    // (the second vector's zero: the kernels write n values)
+    fill_u32(c, mixed ? reinterpret_cast<uint32_t*>(f1.get() + n) : reinterpret_cast<uint32_t*>(d1.get() + n),
+             mixed ? 1 : 2, 0u);
     // the loop keeps A x of its inputs for the final eigenvalue log (the
     // product of the returned u comes from the last iteration)
     DBuf<double> ax;
     if (eig_log && !normLap && !mixed) ax = DBuf<double>(&c.pool, n);
-    StepArgs A[2];
+    // FP32 noise can hold the change of the dot product above a small
+    // tolerance: the mixed form stops after MIXED_ITER_CAP iterations
+    // whatever (the FP64 solve of the finest level follows it)
+    unsigned long long iter_max = 100000000000000ull / (unsigned long long)n;
+    if (mixed && iter_max > MIXED_ITER_CAP) iter_max = MIXED_ITER_CAP;
+    LevelStep A[2];
     c.host_mapped[64] = 0u;  // no kernel of this level has run yet
     for (int k = 0; k < 2; k++) {
-        A[k] = make_args(c, g, plan, wdeg.get(), gb.get(), buf[k], buf[k ^ 1], tol, 0);
-        // FP32 noise can hold the change of the dot product above a small
-        // tolerance: the mixed form stops after MIXED_ITER_CAP iterations
-        // whatever (the FP64 solve of the finest level follows it)
-        if (mixed && A[k].iter_max > MIXED_ITER_CAP) A[k].iter_max = MIXED_ITER_CAP;
-        A[k].hdone = c.host_mapped_dev + 64;
-        A[k].fprev = plan.fsum.get() + NSUM * MAXF_LDS * (k ^ 1);  // sums of the previous launch
-        A[k].fcur = plan.fsum.get() + NSUM * MAXF_LDS * k;
-        A[k].ax = ax.get();
+        A[k] = level_step(c, g, plan, wdeg.get(), gb.get(), buf[k], buf[k ^ 1], tol, 0, k);
+        const auto loop = [&](auto& step) {
+            step.iter_max = iter_max;
+            step.hdone = c.host_mapped_dev + 64;
+            step.ax = ax.get();
+        };
+        if (A[k].by_rows) {
+            loop(A[k].rows);
+            continue;
+        }
+        loop(A[k].stream);
+        A[k].stream.fprev = plan.fsum.get() + NSUM * MAXF_LDS * (k ^ 1);  // sums of the previous launch
+        A[k].stream.fcur = plan.fsum.get() + NSUM * MAXF_LDS * k;
     }
-    run_steps(c, normLap, A);
+    run_steps(c, normLap, A, iter_max);
     MI_HIP(hipStreamSynchronize(c.stream));
     uint32_t flags[2] = {0, 0};
     read_words(c, c.cnt + CT_DONE, flags, 8);

@@ -138,8 +138,58 @@ void build_coarse(Ctx& c, const DGraph& g, const uint32_t* roc, const uint32_t* 
 // block (vrowptr: virtual row q n + r = row r's entries in block q; col_al /
 // w_al hold that order).  Wavefront ranges of pw entries never cross a block:
 // block q holds entries [boff[q], boff[q+1]) and ranges from bwave[q].
+//
+// Levels without rows longer than SHORT_ROW: one launch per iteration, a lane
+// sums a whole row (layout: mi_rows.hip).
+constexpr uint32_t SHORT_ROW = 128;
+struct RowPlan {
+    bool on = false;
+    bool w16 = false;        // 16-bit weights (every weight fits)
+    DBuf<uint32_t> col, w;   // the matrix, slice by slice
+    DBuf<uint32_t> row;      // row of each lane of each slice (INF: none)
+    DBuf<uint32_t> soff;     // first group of each slice
+    DBuf<uint32_t> span;     // first slice of each wavefront
+    DBuf<double> fsum;       // sums of the workgroups, two launches'
+    uint32_t nslices = 0, nblk = 0;
+    uint64_t slots = 0;      // entries with padding
+};
+
+struct RowStep {
+    uint32_t n, wfmt, nblk;
+    const uint32_t* col;
+    const void* w;
+    const uint32_t* row;
+    const uint32_t* soff;
+    const uint32_t* span;
+    const uint32_t* wdeg;
+    const uint32_t* gbp;
+    const double* fprev;     // sums per workgroup, previous launch
+    double* fcur;            // ... this launch
+    const void* yprev;       // n values and a zero, double or float
+    void* ynew;
+    double c, tol;
+    unsigned long long iter_max;
+    int mode;                // 0: loop iteration, 1: one shifted product (a = 0, s = 1), 2: plain A x
+    uint32_t* cnt;
+    int itr, itw;            // the counters of finished iterations that this launch reads and writes
+    double* scal;
+    unsigned long long* niter;
+    uint32_t* hdone;         // done flag in mapped host memory (mode 0 loop), or null
+    double* ax;              // FP64 loop: A x of every iteration's input row by row, or null
+};
+// false: the level has a longer row (nothing is allocated)
+bool plan_rows(Ctx& c, const DGraph& g, RowPlan& p);
+// launches of parity 0 and 1 alternate
+RowStep rows_step(Ctx& c, const DGraph& g, const RowPlan& p, const uint32_t* wdeg, const uint32_t* gb,
+                  const void* yprev, void* ynew, double tol, int mode, int parity);
+void launch_rows(Ctx& c, int normLap, bool f32, const RowStep& A);
+// out = x and the zero that padding reads
+template <class V>
+void pad_copy(Ctx& c, uint32_t n, const double* x, V* out);
+
 constexpr int MAX_COLUMN_BLOCKS = 64;  // LDS column blocks of a level at most
 struct LevelPlan {
+    RowPlan rows;                 // set: the rest is not
     DBuf<uint32_t> rid, wmeta, vrowptr;
     DBuf<uint16_t> rid16, col16;  // 16-bit row offsets; 16-bit columns within a block
     DBuf<uint16_t> w16;           // 16-bit weights when every weight fits

@@ -266,7 +266,7 @@ __device__ __forceinline__ void build_layout(const SmallLevel& V, const SmallJob
             if (j > WAVE || (j == 1 && k > WAVE))
                 __syncthreads();
             else
-                __builtin_amdgcn_wave_barrier();
+                wave_fence();
         }
     }
     __syncthreads();
@@ -462,7 +462,7 @@ __device__ __forceinline__ void share_sums(double (&sum)[3], double* red, bool o
 #pragma unroll
     for (int k = 0; k < 3; k++) sum[k] = wave_sum(sum[k]);
     if (one) {
-        __builtin_amdgcn_wave_barrier();
+        wave_fence();
 #pragma unroll
         for (int k = 0; k < 3; k++) T[k] = sum[k];
         return;
