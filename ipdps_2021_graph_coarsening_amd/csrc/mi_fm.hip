@@ -9,9 +9,9 @@
 // (side, gain bucket, vertex) followed by one pass that links neighbours in
 // that order), the coarsest-level initial partitions (GGGP: one workgroup
 // per start vertex; spectral: the library's power iteration and sort).  The
-// search itself is one wavefront that holds the lists in device memory and
-// makes the reference's moves in the reference's order, with the work of a
-// move spread over the lanes:
+// search itself is one wavefront that holds the lists in LDS, or what does
+// not fit there in device memory, and makes the reference's moves in the
+// reference's order, with the work of a move spread over the lanes:
 //   * the best bucket of a side is found by reading 64 bucket heads per
 //     step, skipping empty stretches with counts of the vertices held per
 //     64 buckets and per 4096 buckets;
@@ -52,24 +52,31 @@ __device__ __forceinline__ void wg_fence()
     __builtin_amdgcn_s_waitcnt(0);
 }
 
-// Loads of the search's state read the L2 (a device-scope access): the
-// words it stores are written through to the L2, and a load that hit an
-// older copy of the line in the vector L1 would return the value from
-// before the store.
+// Loads of words that device-scope atomics change: from the L2, which executes
+// those.
 template <class T>
 __device__ __forceinline__ T ldc(const T* p)
 {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__device__ __forceinline__ long long wave_max_i64(long long v)
+// largest of the lanes' values, in every lane
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v)
 {
-#pragma unroll
-    for (int o = WAVE / 2; o > 0; o >>= 1) {
-        const long long t = __shfl_xor(v, o, WAVE);
-        v = t > v ? t : v;
+    // (a lane without a source keeps its own value)
+#define MI_STEP(CTRL, ROWS)                                                                             \
+    {                                                                                                   \
+        const uint32_t t = (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, ROWS, 0xf, false); \
+        v = t > v ? t : v;                                                                              \
     }
-    return v;
+    MI_STEP(0x111, 0xf)  // row_shr:1, 2, 4, 8: lane 15 of each row of 16 holds the row's
+    MI_STEP(0x112, 0xf)
+    MI_STEP(0x114, 0xf)
+    MI_STEP(0x118, 0xf)
+    MI_STEP(0x142, 0xa)  // row_bcast:15, :31: lane 63 holds all
+    MI_STEP(0x143, 0xc)
+#undef MI_STEP
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, WAVE - 1);
 }
 
 __device__ __forceinline__ long long wave_sum_i64(long long v)
@@ -202,21 +209,139 @@ struct FmSearch {
     uint32_t* order;
     const unsigned long long* acc;
     long long* res;
-    uint32_t n, maxE, NB, NB1, NB2;
+    uint32_t n, m, maxE, NB, NB1, NB2;
 };
+
+constexpr uint32_t FM_BLOCK = 1024;
+
+// Reads `words` words and drops them: they are in this XCD's L2 afterwards.
+__device__ __forceinline__ void touch(const void* p, uint64_t words, uint32_t t, uint32_t step)
+{
+    if (!p) return;
+    const uint32_t* q = static_cast<const uint32_t*>(p);
+    constexpr uint32_t LINE = 32;  // words
+    for (uint64_t i = (uint64_t)t * LINE; i < words; i += (uint64_t)step * LINE) {
+        uint32_t x = q[i];
+        asm volatile("" : "+v"(x));
+    }
+}
+
+// Where the search holds its lists.  Every load of a move depends on the one
+// before, so where the words lie decides its time, besides the some 500
+// instructions of its one wavefront (2d grids, one pass, everything in device
+// memory with waits for every store before, and as here: 60 x 60, 568 moves,
+// all in LDS, 1.90 and 1.23 ms; 400 x 400, 3,717 moves, heads in LDS, 14.6 and
+// 11.4 ms).
+constexpr int FM_GLOBAL = 0;  // everything in device memory, the counts with device-scope atomics
+constexpr int FM_COUNTS = 1;  // the counts in LDS
+constexpr int FM_HEADS = 2;   // ... and the bucket heads
+constexpr int FM_ALL = 3;     // ... and the vertices' records
+constexpr uint32_t FM_LDS_WORDS = 39936;  // 156 KiB
+
+// The lists' words.  One wavefront reads and writes them, and its accesses of
+// one address take place in the order it makes them: words in device memory
+// are read through the vector L1 like any others.  The exception are the
+// counts in device memory, whose atomics the L2 executes; that form reads
+// everything from there and waits for its stores.
+template <int AT>
+struct FmState {
+    const FmSearch& a;
+    uint32_t* sh;  // LDS: counts, heads, records
+    uint32_t c2, hd, rc;
+
+    __device__ __forceinline__ FmState(const FmSearch& a_, uint32_t* sh_) : a(a_), sh(sh_)
+    {
+        c2 = 2 * a.NB1;
+        hd = c2 + 2 * a.NB2;
+        rc = (hd + 2 * a.NB + 3u) & ~3u;
+    }
+    __device__ __forceinline__ void fence() const
+    {
+        if (AT == FM_GLOBAL)
+            wg_fence();
+        else
+            wave_fence();
+    }
+    template <class T>
+    __device__ __forceinline__ T global(const T* p) const
+    {
+        return AT == FM_GLOBAL ? ldc(p) : __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+    }
+    // the lists as the kernels before left them, by the whole workgroup
+    __device__ __forceinline__ void load() const
+    {
+        if (AT == FM_GLOBAL) return;
+        for (uint32_t i = threadIdx.x; i < 2 * a.NB1; i += FM_BLOCK) sh[i] = a.cnt1[i];
+        for (uint32_t i = threadIdx.x; i < 2 * a.NB2; i += FM_BLOCK) sh[c2 + i] = a.cnt2[i];
+        if (AT >= FM_HEADS)
+            for (uint32_t i = threadIdx.x; i < 2 * a.NB; i += FM_BLOCK) sh[hd + i] = a.heads[i];
+        if (AT == FM_ALL)
+            for (uint32_t i = threadIdx.x; i < a.n; i += FM_BLOCK)
+                *reinterpret_cast<uint4*>(&sh[rc + 4 * i]) = a.rec[i];
+        __syncthreads();
+    }
+    __device__ __forceinline__ uint32_t count1(uint32_t i) const { return AT == FM_GLOBAL ? ldc(&a.cnt1[i]) : sh[i]; }
+    __device__ __forceinline__ uint32_t count2(uint32_t i) const
+    {
+        return AT == FM_GLOBAL ? ldc(&a.cnt2[i]) : sh[c2 + i];
+    }
+    // one vertex more (by 1) or less (by -1u) in bucket b of side P
+    __device__ __forceinline__ void count(uint32_t P, uint32_t b, uint32_t by) const
+    {
+        const uint32_t i = P * a.NB1 + (b >> B1), j = P * a.NB2 + (b >> B2);
+        atomicAdd(AT == FM_GLOBAL ? &a.cnt1[i] : &sh[i], by);
+        atomicAdd(AT == FM_GLOBAL ? &a.cnt2[j] : &sh[c2 + j], by);
+    }
+    __device__ __forceinline__ uint32_t head(uint32_t k) const
+    {
+        return AT >= FM_HEADS ? sh[hd + k] : global(&a.heads[k]);
+    }
+    __device__ __forceinline__ void set_head(uint32_t k, uint32_t v) const
+    {
+        if (AT >= FM_HEADS)
+            sh[hd + k] = v;
+        else
+            a.heads[k] = v;
+    }
+    // record words: 0 side | free << 1, 1 gain, 2 previous, 3 next in the bucket
+    __device__ __forceinline__ uint32_t rec(uint32_t v, int k) const
+    {
+        return AT == FM_ALL ? sh[rc + 4 * v + k] : global(reinterpret_cast<const uint32_t*>(a.rec + v) + k);
+    }
+    __device__ __forceinline__ void set_rec(uint32_t v, int k, uint32_t x) const
+    {
+        if (AT == FM_ALL)
+            sh[rc + 4 * v + k] = x;
+        else
+            reinterpret_cast<uint32_t*>(a.rec + v)[k] = x;
+    }
+    __device__ __forceinline__ void set_rec(uint32_t v, uint4 x) const
+    {
+        if (AT == FM_ALL)
+            *reinterpret_cast<uint4*>(&sh[rc + 4 * v]) = x;
+        else
+            a.rec[v] = x;
+    }
+};
+
+// words of LDS that a form needs
+inline uint64_t fm_words(int at, uint64_t n, uint64_t NB, uint64_t NB1, uint64_t NB2)
+{
+    const uint64_t counts = 2 * (NB1 + NB2);
+    return at == FM_COUNTS ? counts : at == FM_HEADS ? counts + 2 * NB : counts + 2 * NB + 3 + 4 * n;
+}
 
 // The highest bucket <= off of side P whose list is not empty, or -1;
 // *head receives its head (NIL for -1).
-__device__ long long fm_top(const FmSearch& a, uint32_t P, long long off, uint32_t* head)
+template <int AT>
+__device__ long long fm_top(const FmState<AT>& st, uint32_t P, long long off, uint32_t* head)
 {
     const int lane = threadIdx.x;
-    const uint32_t* H = a.heads + (size_t)P * a.NB;
-    const uint32_t* C1 = a.cnt1 + (size_t)P * a.NB1;
-    const uint32_t* C2 = a.cnt2 + (size_t)P * a.NB2;
+    const uint32_t H = P * st.a.NB, C1 = P * st.a.NB1, C2 = P * st.a.NB2;
     *head = NIL;
     while (off >= 0) {
         const long long b = off - lane;
-        const uint32_t h = b >= 0 ? ldc(&H[b]) : NIL;
+        const uint32_t h = b >= 0 ? st.head(H + (uint32_t)b) : NIL;
         unsigned long long m = __ballot(h != NIL);
         if (m) {
             const int l = __builtin_ctzll(m);
@@ -227,7 +352,7 @@ __device__ long long fm_top(const FmSearch& a, uint32_t P, long long off, uint32
         if (off < 0) return -1;
         // 64 counts of 64 buckets: the first one below that holds a vertex
         const long long blk = off >> B1, bb = blk - lane;
-        m = __ballot(bb >= 0 && ldc(&C1[bb]) != 0);
+        m = __ballot(bb >= 0 && st.count1(C1 + (uint32_t)bb) != 0);
         if (m) {
             const long long k = blk - (long long)__builtin_ctzll(m);
             if (k < blk) off = (k << B1) + ((1 << B1) - 1);
@@ -236,7 +361,7 @@ __device__ long long fm_top(const FmSearch& a, uint32_t P, long long off, uint32
         off = ((blk - (WAVE - 1)) << B1) - 1;
         if (off < 0) return -1;
         const long long sb = off >> B2, sbb = sb - lane;
-        m = __ballot(sbb >= 0 && ldc(&C2[sbb]) != 0);
+        m = __ballot(sbb >= 0 && st.count2(C2 + (uint32_t)sbb) != 0);
         if (m) {
             const long long k = sb - (long long)__builtin_ctzll(m);
             if (k < sb) off = (k << B2) + ((1 << B2) - 1);
@@ -266,13 +391,28 @@ __device__ __forceinline__ uint32_t rdl(uint32_t v, int l) { return (uint32_t)__
 // adjacent leaving vertices is walked lane to lane, and the stores of the
 // removals and insertions of one step go to distinct words.  Every step
 // begins by waiting for the previous step's stores.
-__global__ void __launch_bounds__(WAVE) k_fm_search(FmSearch a)
+template <int AT>
+__global__ void __launch_bounds__(FM_BLOCK) k_fm_search(FmSearch a)
 {
+    __shared__ alignas(16) uint32_t sh[AT == FM_GLOBAL ? 4 : FM_LDS_WORDS];
+    const FmState<AT> st(a, sh);
+    st.load();
+    if (threadIdx.x >= WAVE) {
+        // Each XCD has read its part of the graph before: a first read by the
+        // search would go past this one's L2.  (The search has begun
+        // meanwhile; 5 % of a pass.)
+        const uint32_t t = threadIdx.x - WAVE, step = FM_BLOCK - WAVE;
+        if (AT != FM_ALL) touch(a.rec, 4ull * a.n, t, step);
+        touch(a.rowptr, (uint64_t)a.n + 1, t, step);
+        touch(a.vtx_w, a.n, t, step);
+        touch(a.col, a.m, t, step);
+        touch(a.w, a.m, t, step);
+        return;
+    }
     const int lane = threadIdx.x;
     const unsigned long long lt = lane ? (~0ull >> (WAVE - lane)) : 0ull;
     const long long maxE = a.maxE;
     const uint32_t NB = a.NB;
-    uint32_t* R32 = reinterpret_cast<uint32_t*>(a.rec);
     long long cut = (long long)a.acc[0];
     long long balance = (long long)a.acc[1];
     const long long start_bal = balance < 0 ? -balance : balance;
@@ -286,13 +426,13 @@ __global__ void __launch_bounds__(WAVE) k_fm_search(FmSearch a)
     uint32_t hd0 = NIL, hd1 = NIL;
     bool scan0 = true, scan1 = true;
     for (;;) {
-        wg_fence();
+        st.fence();
         if (scan0 || hd0 == NIL) {
-            if (off0 >= 0) off0 = fm_top(a, 0, off0, &hd0);
+            if (off0 >= 0) off0 = fm_top<AT>(st, 0, off0, &hd0);
             scan0 = false;
         }
         if (scan1 || hd1 == NIL) {
-            if (off1 >= 0) off1 = fm_top(a, 1, off1, &hd1);
+            if (off1 >= 0) off1 = fm_top<AT>(st, 1, off1, &hd1);
             scan1 = false;
         }
         const bool has0 = hd0 != NIL, has1 = hd1 != NIL;
@@ -315,17 +455,16 @@ __global__ void __launch_bounds__(WAVE) k_fm_search(FmSearch a)
             bad = 2;
             break;
         }
-        const uint32_t ns = ldc(&R32[4 * (size_t)s + 3]);
+        const uint32_t ns = st.rec(s, 3);
         const uint32_t vw = a.vtx_w ? a.vtx_w[s] : 1u;
         const uint32_t r0 = a.rowptr[s], r1 = a.rowptr[s + 1];
         const uint32_t sp = P ^ 1u;  // the side s moves to
         if (lane == 0) {
-            a.heads[key] = ns;
-            if (ns != NIL) R32[4 * (size_t)ns + 2] = NIL;
-            R32[4 * (size_t)s] = sp;  // moved, no longer free
+            st.set_head(key, ns);
+            if (ns != NIL) st.set_rec(ns, 2, NIL);
+            st.set_rec(s, 0, sp);  // moved, no longer free
             a.order[total] = s;
-            atomicSub(&a.cnt1[P * a.NB1 + ((uint32_t)top >> B1)], 1u);
-            atomicSub(&a.cnt2[P * a.NB2 + ((uint32_t)top >> B2)], 1u);
+            st.count(P, (uint32_t)top, 0u - 1u);
         }
         if (P)
             hd1 = ns;
@@ -356,7 +495,8 @@ __global__ void __launch_bounds__(WAVE) k_fm_search(FmSearch a)
             // a row that names a vertex twice within these 64 entries is
             // taken one entry at a time (the reference's order)
             unsigned long long pend = __ballot(valid), dup = 0;
-            {
+            const uint32_t vb = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x138, 0xf, 0xf, false);  // lane - 1's
+            if (__ballot(valid && lane && v <= vb)) {  // (none in a row in column order)
                 unsigned long long todo = pend;
                 while (todo) {
                     const int l = __builtin_ctzll(todo);
@@ -370,14 +510,13 @@ __global__ void __launch_bounds__(WAVE) k_fm_search(FmSearch a)
                 const unsigned long long step = dup ? (pend & (~pend + 1)) : pend;
                 pend &= ~step;
                 const bool mine = (step >> lane) & 1ull;
-                wg_fence();
+                st.fence();
                 uint32_t sv = 0, gv = 0, pn = NIL, nn = NIL;
                 if (mine) {
-                    const uint32_t* r = &R32[4 * (size_t)v];
-                    sv = ldc(r);
-                    gv = ldc(r + 1);
-                    pn = ldc(r + 2);
-                    nn = ldc(r + 3);
+                    sv = st.rec(v, 0);
+                    gv = st.rec(v, 1);
+                    pn = st.rec(v, 2);
+                    nn = st.rec(v, 3);
                 }
                 const bool act = mine && (sv & 2u);
                 const int32_t og = (int32_t)gv;
@@ -436,7 +575,11 @@ __global__ void __launch_bounds__(WAVE) k_fm_search(FmSearch a)
                 const unsigned long long above = grp & ~lt & ~(1ull << lane);
                 const int lo = below ? 63 - __builtin_clzll(below) : lane;
                 const int hi = above ? __builtin_ctzll(above) : lane;
-                const uint32_t vlo = __shfl(v, lo, WAVE), vhi = __shfl(v, hi, WAVE);
+                uint32_t vlo = v, vhi = v;
+                if (__ballot((below | above) != 0)) {
+                    vlo = __shfl(v, lo, WAVE);
+                    vhi = __shfl(v, hi, WAVE);
+                }
                 // the old head of each target bucket: where a run left from
                 // the head of that bucket, the vertex after the run; else
                 // the stored head.  A run leaving from the head of a bucket
@@ -455,30 +598,28 @@ __global__ void __launch_bounds__(WAVE) k_fm_search(FmSearch a)
                     const bool hit = __ballot(act && nkey == kl) != 0;
                     if (lane == l) ins_here = hit;
                 }
-                if (act && !ohk) oh = ldc(&a.heads[nkey]);
+                if (act && !ohk) oh = st.head(nkey);
                 if (first) {
                     if (pn == NIL) {
                         if (!ins_here) {
-                            a.heads[okey] = q;
-                            if (q != NIL) R32[4 * (size_t)q + 2] = NIL;
+                            st.set_head(okey, q);
+                            if (q != NIL) st.set_rec(q, 2, NIL);
                         }
                     } else {
-                        R32[4 * (size_t)pn + 3] = q;
-                        if (q != NIL) R32[4 * (size_t)q + 2] = pn;
+                        st.set_rec(pn, 3, q);
+                        if (q != NIL) st.set_rec(q, 2, pn);
                     }
                 }
                 if (act) {
-                    atomicSub(&a.cnt1[pv * a.NB1 + (ob >> B1)], 1u);
-                    atomicSub(&a.cnt2[pv * a.NB2 + (ob >> B2)], 1u);
-                    a.rec[v] = make_uint4(sv, (uint32_t)ng, above ? vhi : NIL, below ? vlo : oh);
-                    if (!below && oh < a.n) R32[4 * (size_t)oh + 2] = v;
-                    if (!above) a.heads[nkey] = v;
-                    atomicAdd(&a.cnt1[pv * a.NB1 + (nb >> B1)], 1u);
-                    atomicAdd(&a.cnt2[pv * a.NB2 + (nb >> B2)], 1u);
+                    st.count(pv, ob, 0u - 1u);
+                    st.set_rec(v, make_uint4(sv, (uint32_t)ng, above ? vhi : NIL, below ? vlo : oh));
+                    if (!below && oh < a.n) st.set_rec(oh, 2, v);
+                    if (!above) st.set_head(nkey, v);
+                    st.count(pv, nb, 1u);
                 }
                 // each side's highest bucket and its head
                 {
-                    const long long bi = wave_max_i64(act && pv == 0 ? (long long)nb : -1);
+                    const long long bi = (long long)wave_max_u32(act && pv == 0 ? nb + 1 : 0u) - 1;
                     if (bi >= 0 && bi >= off0) {
                         const unsigned long long hl = __ballot(act && pv == 0 && (long long)nb == bi && !above);
                         off0 = bi;
@@ -489,7 +630,7 @@ __global__ void __launch_bounds__(WAVE) k_fm_search(FmSearch a)
                     }
                 }
                 {
-                    const long long bi = wave_max_i64(act && pv == 1 ? (long long)nb : -1);
+                    const long long bi = (long long)wave_max_u32(act && pv == 1 ? nb + 1 : 0u) - 1;
                     if (bi >= 0 && bi >= off1) {
                         const unsigned long long hl = __ballot(act && pv == 1 && (long long)nb == bi && !above);
                         off1 = bi;
@@ -504,11 +645,15 @@ __global__ void __launch_bounds__(WAVE) k_fm_search(FmSearch a)
         }
         if (bad || counter > 500) break;
     }
-    wg_fence();
+    st.fence();
     // undo the moves after the kept prefix (:1222-1233)
     for (uint32_t i = (uint32_t)(argmin + 1) + lane; i < total; i += WAVE) {
-        const uint32_t s = a.order[i];
-        R32[4 * (size_t)s] = ldc(&R32[4 * (size_t)s]) ^ 1u;
+        const uint32_t s = st.global(&a.order[i]);
+        st.set_rec(s, 0, st.rec(s, 0) ^ 1u);
+    }
+    if (AT == FM_ALL) {
+        st.fence();
+        for (uint32_t i = lane; i < a.n; i += WAVE) a.rec[i].x = st.rec(i, 0);
     }
     if (lane == 0) {
         a.res[0] = min_cut;
@@ -740,11 +885,21 @@ uint32_t fm_pass(Ctx& c, FmLevel& L, long long* info)
     a.acc = L.acc.get();
     a.res = reinterpret_cast<long long*>(L.acc.get() + 2);
     a.n = n;
+    a.m = (uint32_t)g.m;
     a.maxE = L.maxE;
     a.NB = L.NB;
     a.NB1 = L.NB1;
     a.NB2 = L.NB2;
-    k_fm_search<<<1, WAVE, 0, c.stream>>>(a);
+    // as much of the lists in LDS as fits
+    const auto fits = [&](int at) { return fm_words(at, n, L.NB, L.NB1, L.NB2) <= FM_LDS_WORDS; };
+    if (fits(FM_ALL))
+        k_fm_search<FM_ALL><<<1, FM_BLOCK, 0, c.stream>>>(a);
+    else if (fits(FM_HEADS))
+        k_fm_search<FM_HEADS><<<1, FM_BLOCK, 0, c.stream>>>(a);
+    else if (fits(FM_COUNTS))
+        k_fm_search<FM_COUNTS><<<1, FM_BLOCK, 0, c.stream>>>(a);
+    else
+        k_fm_search<FM_GLOBAL><<<1, FM_BLOCK, 0, c.stream>>>(a);
     MI_HIP(hipGetLastError());
     long long res[5] = {0, 0, 0, 0, 0};
     read_words(c, L.acc.get() + 2, res, sizeof(res));

@@ -332,7 +332,7 @@ __device__ __forceinline__ void leave_sums(const RowStep& A, const double (&S)[N
 // Bound by memory on large levels and by the chain counter, sums, entries,
 // gathers on small ones (one launch is not shorter than about 7 us).  us per
 // iteration, the streaming step's two launches before and this one: 3d grid
-// 128^3 in FP64 73 and 47 (2.9 TB/s of the layout and vectors; the gathers of
+// 128^3 in FP64 73 and 47 (2.2 TB/s of the layout and vectors; the gathers of
 // neighbours a plane away miss L1), its level of 628,115 vertices 44 and 35,
 // random geometric graph of 150,000 vertices 37 and 28, 12,882 vertices 15.9
 // and 11.4.

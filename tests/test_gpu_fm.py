@@ -223,3 +223,15 @@ def test_partition_4way_fm_vs_oracle(ctx, name):
     exp[~side] = o0["part"]
     exp[side] = 2 + o1["part"]
     assert np.array_equal(r4.part, exp)
+
+
+@pytest.mark.parametrize("n,wt", [
+    (9979, 1), (9980, 1),  # the lists and the vertices' records fill 156 KiB of LDS, or do not fit
+    (500, 4910), (500, 4914),  # ... the bucket heads
+    (500, 314500), (500, 314600)])  # ... the counts of 64 buckets
+def test_fm_lists_at_the_edge_of_lds(ctx, n, wt):
+    rp, col = graphs.path(n)[:2]
+    w = np.full(len(col), wt, np.uint32)
+    rng = np.random.default_rng(n + wt)
+    for part in (rng.random(n) < 0.5, np.arange(n) < n // 3):
+        _check_refine(ctx, rp, col, w, None, part.astype(np.uint8))
