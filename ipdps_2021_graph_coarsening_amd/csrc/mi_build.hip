@@ -1290,14 +1290,29 @@ __global__ void k_cc_union(uint64_t m, const uint32_t* __restrict__ rowptr, cons
     }
 }
 
-// roots, component sizes, and the largest (size, smallest root) as one key
-__global__ void k_cc_roots(uint32_t n, uint32_t* __restrict__ parent, uint32_t* __restrict__ size)
+// roots and component sizes.  Nearly all vertices of a graph tend to share a
+// root, whose counter would take one atomic each (8.9 million vertices: 100
+// ms): a workgroup counts the vertices that have its first one's root and adds
+// them at once.
+__global__ void __launch_bounds__(BLOCK) k_cc_roots(uint32_t n, uint32_t* __restrict__ parent,
+                                                    uint32_t* __restrict__ size)
 {
-    const uint32_t i = blockIdx.x * BLOCK + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t r = cc_find(parent, i);
-    parent[i] = r;
-    atomicAdd(&size[r], 1u);
+    __shared__ uint32_t lds[BLOCK / WAVE], common;
+    const uint32_t step = gridDim.x * BLOCK;
+    if (threadIdx.x == 0) common = cc_find(parent, blockIdx.x * BLOCK);
+    __syncthreads();
+    const uint32_t rc = common;
+    uint32_t mine = 0;
+    for (uint64_t i = blockIdx.x * BLOCK + threadIdx.x; i < n; i += step) {
+        const uint32_t r = cc_find(parent, (uint32_t)i);
+        __hip_atomic_store(&parent[i], r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (r == rc)
+            mine++;
+        else
+            atomicAdd(&size[r], 1u);
+    }
+    mine = block_sum_u32(mine, lds);
+    if (threadIdx.x == 0 && mine) atomicAdd(&size[rc], mine);
 }
 
 __global__ void k_cc_largest(uint32_t n, const uint32_t* __restrict__ size, unsigned long long* __restrict__ best)
@@ -1380,7 +1395,8 @@ void graph_from_edges(Ctx& c, uint32_t n, uint64_t ne, const uint32_t* du, const
         k_cc_union<<<grid1(g.m), BLOCK, 0, c.stream>>>(g.m, g.R(), roc.get(), g.Cc(), parent.get());
         MI_HIP(hipGetLastError());
     }
-    k_cc_roots<<<grid1(n), BLOCK, 0, c.stream>>>(n, parent.get(), size.get());
+    // (every workgroup begins inside the graph)
+    k_cc_roots<<<std::min(grid1(n), 1024u), BLOCK, 0, c.stream>>>(n, parent.get(), size.get());
     MI_HIP(hipGetLastError());
     DBuf<unsigned long long> best(&c.pool, 1);
     fill_u32(c, reinterpret_cast<uint32_t*>(best.get()), 2, 0u);
