@@ -418,7 +418,8 @@ bool plan_rows(Ctx& c, const DGraph& g, RowPlan& p)
         DBuf<uint32_t> x(&c.pool, 2);
         fill_u32(c, x.get(), 2, 0u);
         const uint64_t work = std::max<uint64_t>(n, weights ? m : 0);
-        k_extremes<<<(unsigned)std::min<uint64_t>(8ull * ncu, ceil_div(work, BLOCK)), BLOCK, 0, c.stream>>>(
+        // (two atomics per workgroup on the same words: few workgroups)
+        k_extremes<<<(unsigned)std::min<uint64_t>(ncu, ceil_div(work, 4 * BLOCK)), BLOCK, 0, c.stream>>>(
             n, m, g.R(), weights ? g.W() : nullptr, x.get());
         MI_HIP(hipGetLastError());
         read_words(c, x.get(), ext, 8);
