@@ -272,6 +272,7 @@ void build_hierarchy(Ctx& c, const DGraph& g, uint64_t seed, std::vector<DLevel>
     lv.reserve(MI_MAX_LEVELS + 1);
     lv.push_back(borrow_level(c, g));
     HecTimes ht;
+    HecStream stream;
     double build_ms = 0;
     int level = 0;
     while (lv.back().g.n > 50u) {  // SGPAR_COARSENING_VTX_CUTOFF, definitions_kokkos.h:77-79
@@ -281,7 +282,7 @@ void build_hierarchy(Ctx& c, const DGraph& g, uint64_t seed, std::vector<DLevel>
         DBuf<uint32_t> roc;
         build_row_index(c, a.g, roc);
         const uint32_t nc =
-            hec_map(c, a.g, roc.get(), level, seed, a.vcmap.get(), nullptr, nullptr, st ? &ht : nullptr);
+            hec_map(c, a.g, roc.get(), level, seed, a.vcmap.get(), nullptr, nullptr, st ? &ht : nullptr, &stream);
         a.nc_next = nc;
         DLevel nl;
         auto tb = std::chrono::steady_clock::now();

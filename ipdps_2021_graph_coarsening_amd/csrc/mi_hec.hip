@@ -88,6 +88,61 @@ __global__ void k_scatter_pos(const uint32_t* __restrict__ vperm, uint32_t n, ui
     if (i < n) pos[vperm[i]] = i;
 }
 
+// The permutation of the first n vertices from that of more: every level of a
+// hierarchy draws from the same seed, so a coarser level's keys are the first
+// of the finer level's and its argsort is that one without the vertices from n
+// on.  Workgroup b takes PERM_CH entries; k_perm_filter sums the counts of the
+// workgroups before it (at most a few thousand) itself.
+constexpr uint32_t PERM_CH = 8 * BLOCK;
+__global__ void __launch_bounds__(BLOCK) k_perm_count(uint32_t np, const uint32_t* __restrict__ prev, uint32_t n,
+                                                      uint32_t* __restrict__ counts)
+{
+    __shared__ uint32_t lds[BLOCK / WAVE];
+    const uint64_t i0 = (uint64_t)blockIdx.x * PERM_CH;
+    uint32_t k = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < PERM_CH / BLOCK; j++) {
+        const uint64_t i = i0 + j * BLOCK + threadIdx.x;
+        k += i < np && prev[i] < n ? 1u : 0u;
+    }
+    k = block_sum_u32(k, lds);
+    if (threadIdx.x == 0) counts[blockIdx.x] = k;
+}
+
+__global__ void __launch_bounds__(BLOCK) k_perm_filter(uint32_t np, const uint32_t* __restrict__ prev, uint32_t n,
+                                                       const uint32_t* __restrict__ counts,
+                                                       uint32_t* __restrict__ vperm, uint32_t* __restrict__ pos)
+{
+    __shared__ uint32_t lds[BLOCK / WAVE], base, wcnt[BLOCK / WAVE];
+    uint32_t before = 0;
+    for (uint32_t b = threadIdx.x; b < blockIdx.x; b += BLOCK) before += counts[b];
+    before = block_sum_u32(before, lds);
+    if (threadIdx.x == 0) base = before;
+    // a wavefront takes consecutive entries, 64 at a time
+    constexpr uint32_t STEPS = PERM_CH / BLOCK;
+    const uint32_t lane = threadIdx.x & (WAVE - 1), wv = threadIdx.x / WAVE;
+    const uint64_t i0 = (uint64_t)blockIdx.x * PERM_CH + wv * (WAVE * STEPS) + lane;
+    uint32_t v[STEPS], k = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < STEPS; j++) v[j] = i0 + j * WAVE < np ? prev[i0 + j * WAVE] : INF;
+#pragma unroll
+    for (uint32_t j = 0; j < STEPS; j++) k += (uint32_t)__popcll(__ballot(v[j] < n));
+    if (lane == 0) wcnt[wv] = k;
+    __syncthreads();
+    uint32_t at = base;
+    for (uint32_t j = 0; j < wv; j++) at += wcnt[j];
+#pragma unroll
+    for (uint32_t j = 0; j < STEPS; j++) {
+        const unsigned long long in = __ballot(v[j] < n);
+        if (v[j] < n) {
+            const uint32_t r = at + (uint32_t)__popcll(in & ((1ull << lane) - 1ull));
+            vperm[r] = v[j];
+            pos[v[j]] = r;
+        }
+        at += (uint32_t)__popcll(in);
+    }
+}
+
 // level 1: hn(i) = col[rowptr[i] + draw % deg], isolated: draw % n
 __global__ void k_hn_random(uint32_t n, const uint32_t* __restrict__ rowptr,
                             const uint32_t* __restrict__ col, const uint64_t* __restrict__ draws,
@@ -2208,7 +2263,7 @@ static uint32_t map_closed_form(Ctx& c, uint32_t n, const uint32_t* vperm, const
 }
 
 uint32_t hec_map(Ctx& c, const DGraph& g, const uint32_t* roc, int level, uint64_t seed, uint32_t* vcmap,
-                 uint32_t* vperm_out, uint32_t* hn_out, HecTimes* t)
+                 uint32_t* vperm_out, uint32_t* hn_out, HecTimes* t, HecStream* keep)
 {
     const uint32_t n = g.n;
     MI_CHECK(n > 0, ST_ARG, "empty level");
@@ -2224,21 +2279,36 @@ uint32_t hec_map(Ctx& c, const DGraph& g, const uint32_t* roc, int level, uint64
         for (auto& e : ev) MI_HIP(hipEventCreate(&e));
     if (t) MI_HIP(hipEventRecord(ev[0], c.stream));
 
-    // ---- random stream: positions [0, 2n)
-    DBuf<uint64_t> draws(&c.pool, 2ull * n);
-    xs_draws(c, xs_pool_state(seed), 0, 2ull * n, draws.get());
-
-    // ---- permutation: argsort of the first n draws
-    DBuf<uint64_t> keys(&c.pool, n), ktmp(&c.pool, n);
-    DBuf<uint32_t> vperm(&c.pool, n), vtmp(&c.pool, n), pos(&c.pool, n);
-    MI_HIP(hipMemcpyAsync(keys.get(), draws.get(), (size_t)n * 8, hipMemcpyDeviceToDevice, c.stream));
-    iota_u32(c, vperm.get(), n, 0);
-    sort_random_keys(c, keys.get(), vperm.get(), n, ktmp.get(), vtmp.get());
-    k_scatter_pos<<<grid1(n), BLOCK, 0, c.stream>>>(vperm.get(), n, pos.get());
-    MI_HIP(hipGetLastError());
-    keys.reset();
-    ktmp.reset();
-    vtmp.reset();
+    // ---- random stream: positions [0, 2n); permutation: argsort of the first
+    // n draws.  Both from the finer level's where the caller keeps them.
+    HecStream own;
+    HecStream& hs = keep ? *keep : own;
+    DBuf<uint32_t> pos(&c.pool, n);
+    if (hs.n && hs.seed == seed && n <= hs.n) {
+        DBuf<uint32_t> next(&c.pool, n);
+        const uint32_t nb = (uint32_t)ceil_div(hs.n, PERM_CH);
+        DBuf<uint32_t> counts(&c.pool, nb);
+        k_perm_count<<<nb, BLOCK, 0, c.stream>>>(hs.n, hs.vperm.get(), n, counts.get());
+        MI_HIP(hipGetLastError());
+        k_perm_filter<<<nb, BLOCK, 0, c.stream>>>(hs.n, hs.vperm.get(), n, counts.get(), next.get(), pos.get());
+        MI_HIP(hipGetLastError());
+        hs.vperm = std::move(next);
+    } else {
+        hs.draws = DBuf<uint64_t>(&c.pool, 2ull * n);
+        xs_draws(c, xs_pool_state(seed), 0, 2ull * n, hs.draws.get());
+        hs.vperm = DBuf<uint32_t>(&c.pool, n);
+        DBuf<uint64_t> keys(&c.pool, n), ktmp(&c.pool, n);
+        DBuf<uint32_t> vtmp(&c.pool, n);
+        MI_HIP(hipMemcpyAsync(keys.get(), hs.draws.get(), (size_t)n * 8, hipMemcpyDeviceToDevice, c.stream));
+        iota_u32(c, hs.vperm.get(), n, 0);
+        sort_random_keys(c, keys.get(), hs.vperm.get(), n, ktmp.get(), vtmp.get());
+        k_scatter_pos<<<grid1(n), BLOCK, 0, c.stream>>>(hs.vperm.get(), n, pos.get());
+        MI_HIP(hipGetLastError());
+        hs.seed = seed;
+    }
+    hs.n = n;
+    const DBuf<uint64_t>& draws = hs.draws;
+    const DBuf<uint32_t>& vperm = hs.vperm;
     if (t) MI_HIP(hipEventRecord(ev[1], c.stream));
 
     // ---- heavy neighbour (matching: the first heaviest; no row may be empty)
@@ -2272,7 +2342,7 @@ uint32_t hec_map(Ctx& c, const DGraph& g, const uint32_t* roc, int level, uint64
         k_hn_iso<<<grid1(n), BLOCK, 0, c.stream>>>(n, iso.get(), rank.get(), draws.get(), hn.get());
         MI_HIP(hipGetLastError());
     }
-    draws.reset();
+    own.draws.reset();
     if (t) MI_HIP(hipEventRecord(ev[2], c.stream));
 
     if (matching) {

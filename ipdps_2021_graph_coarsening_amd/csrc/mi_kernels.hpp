@@ -39,6 +39,15 @@ struct HecTimes {
     double permute_ms = 0, heavy_ms = 0, map_ms = 0, build_ms = 0;
 };
 
+// The draws and the permutation of a level, from which the coarser levels of
+// the same hierarchy take theirs (the seed is the same on every level).
+struct HecStream {
+    uint64_t seed = 0;
+    uint32_t n = 0;          // vertices of vperm
+    DBuf<uint64_t> draws;    // positions [0, 2 n) of the finest level
+    DBuf<uint32_t> vperm;
+};
+
 // ---------------------------------------------------------------- row index
 // roc[k] = row holding entry 64 k (k < ceil(m / 64)), roc[ceil(m/64)] = n - 1.
 // Lets a lane find the row of any entry with a search over a short range.
@@ -119,7 +128,7 @@ void xs_draws(Ctx& c, uint64_t state0, uint64_t first, uint64_t count, uint64_t*
 // returns nc.  level >= 1 as in heuristics.h:930 (level 1 = random neighbour).
 // roc is the row index of g (build_row_index).
 uint32_t hec_map(Ctx& c, const DGraph& g, const uint32_t* roc, int level, uint64_t seed, uint32_t* vcmap,
-                 uint32_t* vperm_out, uint32_t* hn_out, HecTimes* t);
+                 uint32_t* vperm_out, uint32_t* hn_out, HecTimes* t, HecStream* keep = nullptr);
 
 // Coarse graph P^T A P without diagonal, rows sorted, duplicates merged.
 // The reference converter's graph from an edge list on the device (u, v, w

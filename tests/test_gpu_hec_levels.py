@@ -1,0 +1,35 @@
+"""The maps of a hierarchy against the same levels coarsened one by one: a
+hierarchy draws the random stream once and filters each level's permutation
+out of the finer level's (csrc/mi_hec.hip, 2048 entries per workgroup), a
+single level draws and sorts its own.  Integers, compared exactly; each
+hierarchy's own levels against the oracle: test_gpu_parity.py."""
+import numpy as np
+import pytest
+
+from ipdps_2021_graph_coarsening_amd import graphs
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("variant", [0, 1, 3, 4])
+@pytest.mark.parametrize("n", [51, 255, 2047, 2048, 2049, 4097, 70001])
+def test_levels_one_by_one(ctx, n, variant):
+    rng = np.random.default_rng(n)
+    k = np.arange(n - 1)
+    u, v = np.concatenate([k, rng.integers(0, n, n)]), np.concatenate([k + 1, rng.integers(0, n, n)])
+    rp, col, w = graphs.from_edges(n, u, v, rng.integers(1, 9, len(u)), lcc=False)
+    ctx.set_coarsening(variant)
+    try:
+        g = ctx.graph(rp, col, w)
+        H = g.hierarchy(5)
+        assert H.nlevels > 1
+        for l in range(H.nlevels - 1):
+            a = H.level(l)
+            one = ctx.graph(a["rowptr"], a["col"], a["w"])
+            vcmap = one.hec_level(l + 1, 5)[0]
+            one.close()
+            assert np.array_equal(vcmap, a["vcmap"])
+        H.close()
+        g.close()
+    finally:
+        ctx.set_coarsening(0)
