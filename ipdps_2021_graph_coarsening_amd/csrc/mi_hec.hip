@@ -980,6 +980,181 @@ __global__ void k_match_compact(uint32_t len, const uint32_t* __restrict__ list,
     if (k < len && keep[k]) next[at[k]] = list[k];
 }
 
+// The rounds over a list of at most MATCH_ONE_WG slots to their end, in one
+// workgroup: the phases of the kernels above with a barrier where those end,
+// so the result is theirs.  A round by launches costs some twelve of them and a
+// wait of the host per step, about 110 us however short the list (the maps of
+// all 15 levels of a random geometric graph of 150,001 vertices: 6.2 ms by
+// launches, 3.5 ms so).  LANES lanes share the row of a slot when it looks for
+// its next neighbour.
+constexpr uint32_t MATCH_ONE_WG = 4096;
+constexpr int MATCH_BLOCK = 1024;
+
+struct MatchTail {
+    uint32_t len, nc, cap;  // cap: rounds at most
+    int swap, idle, level;
+    const uint32_t* rowptr;
+    const uint32_t* col;
+    const uint32_t* w;
+    const uint32_t* pos;
+    uint32_t* la;
+    uint32_t* lb;
+    uint32_t* hn;
+    uint32_t* vcmap;
+    uint8_t* est;
+    uint32_t* first;
+    uint32_t* keep;
+    uint32_t* out;  // ids given, swap, 0 or what went wrong (1: only self-loops left, 2: did not end)
+};
+
+template <int LANES>
+__global__ void __launch_bounds__(MATCH_BLOCK) k_match_tail(MatchTail a)
+{
+    __shared__ uint32_t wsum[2][MATCH_BLOCK / WAVE], undecided;
+    const uint32_t t = threadIdx.x, lane = t & (WAVE - 1), wv = t / WAVE;
+    uint32_t len = a.len, nc = a.nc, err = 0;
+    int swap = a.swap, idle = a.idle;
+    uint32_t *la = a.la, *lb = a.lb;
+    // rank of a flag among the workgroup's, thread by thread, and their number
+    int turn = 0;
+    const auto ranked = [&](bool f, uint32_t& all) {
+        const unsigned long long b = __ballot(f);
+        if (lane == 0) wsum[turn][wv] = (uint32_t)__popcll(b);
+        __syncthreads();
+        uint32_t before = 0;
+        all = 0;
+        for (uint32_t j = 0; j < MATCH_BLOCK / WAVE; j++) {
+            before += j < wv ? wsum[turn][j] : 0u;
+            all += wsum[turn][j];
+        }
+        turn ^= 1;  // (the next call's counts go elsewhere: one barrier per call)
+        return before + (uint32_t)__popcll(b & ((1ull << lane) - 1ull));
+    };
+    for (uint32_t round = 0; len > 0; round++) {
+        if (round > a.cap) {
+            err = 2;
+            break;
+        }
+        if (t == 0) undecided = 0;
+        __syncthreads();
+        for (uint32_t k = t; k < len; k += MATCH_BLOCK) {
+            const uint32_t u = la[k], v = a.hn[u];
+            const int cond = a.pos[u] < a.pos[v] ? 1 : 0;
+            const bool in = (cond ^ swap) && u != v && a.vcmap[v] == INF;
+            a.est[k] = in ? 1 : 0;
+            if (in) undecided = 1;
+        }
+        __syncthreads();
+        // (every step with an undecided edge takes one: at most len steps)
+        uint32_t step = 0;
+        for (; undecided && step <= len; step++) {
+            for (uint32_t k = t; k < len; k += MATCH_BLOCK) {
+                if (a.est[k] != 1) continue;
+                const uint32_t u = la[k];
+                atomicMin(&a.first[u], k);
+                atomicMin(&a.first[a.hn[u]], k);
+            }
+            __syncthreads();
+            if (t == 0) undecided = 0;
+            for (uint32_t k = t; k < len; k += MATCH_BLOCK) {
+                if (a.est[k] != 1) continue;
+                const uint32_t u = la[k], v = a.hn[u];
+                // (the L2 holds what the atomics left)
+                if (__hip_atomic_load(&a.first[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == k &&
+                    __hip_atomic_load(&a.first[v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == k) {
+                    a.est[k] = 2;
+                    a.vcmap[u] = PENDING;
+                    a.vcmap[v] = PENDING;
+                }
+            }
+            __syncthreads();
+            for (uint32_t k = t; k < len; k += MATCH_BLOCK) {
+                const uint8_t s = a.est[k];
+                if (s == 0) continue;
+                const uint32_t u = la[k], v = a.hn[u];
+                a.first[u] = INF;
+                a.first[v] = INF;
+                if (s != 1) continue;
+                if (a.vcmap[u] != INF || a.vcmap[v] != INF)
+                    a.est[k] = 0;
+                else
+                    undecided = 1;
+            }
+            __syncthreads();
+        }
+        if (step > len) {
+            err = 2;
+            break;
+        }
+        uint32_t pairs = 0, all;
+        for (uint32_t k0 = 0; k0 < len; k0 += MATCH_BLOCK) {
+            const uint32_t k = k0 + t;
+            const bool taken = k < len && a.est[k] == 2;
+            const uint32_t id = nc + pairs + ranked(taken, all);
+            if (taken) {
+                const uint32_t u = la[k];
+                a.vcmap[u] = id;
+                a.vcmap[a.hn[u]] = id;
+            }
+            pairs += all;
+        }
+        nc += pairs;
+        __syncthreads();
+        for (uint32_t k = t / LANES; k < len; k += MATCH_BLOCK / LANES) {
+            const uint32_t u = la[k], l = t % LANES;
+            const bool open = a.vcmap[u] == INF;
+            uint64_t key = 0;
+            bool any = false;
+            if (open) {
+                for (uint32_t e = a.rowptr[u] + l, r1 = a.rowptr[u + 1]; e < r1; e += LANES) {
+                    const uint32_t v = a.col[e];
+                    if (a.vcmap[v] != INF) continue;
+                    const uint32_t kv = a.level == 1 ? a.pos[v] : (a.w ? a.w[e] : 1u);
+                    const uint64_t x = ((uint64_t)kv << 32) | e;
+                    key = (!any || x > key) ? x : key;
+                    any = true;
+                }
+            }
+            // (key + 1 below: 0 says none; e < 2^32 - 1 keeps it from wrapping)
+            uint64_t best = any ? key + 1 : 0;
+#pragma unroll
+            for (int o = LANES / 2; o > 0; o >>= 1) {
+                const uint64_t x = __shfl_xor(best, o, WAVE);
+                best = x > best ? x : best;
+            }
+            if (l == 0) {
+                a.keep[k] = best ? 1u : 0u;
+                if (best) a.hn[u] = a.col[(uint32_t)(best - 1)];
+            }
+        }
+        __syncthreads();
+        uint32_t next = 0;
+        for (uint32_t k0 = 0; k0 < len; k0 += MATCH_BLOCK) {
+            const uint32_t k = k0 + t;
+            const bool stays = k < len && a.keep[k];
+            const uint32_t at = next + ranked(stays, all);
+            if (stays) lb[at] = la[k];
+            next += all;
+        }
+        idle = pairs ? 0 : idle + 1;
+        if (idle >= 3 && next > 0) {
+            err = 1;
+            break;
+        }
+        len = next;
+        swap ^= 1;
+        uint32_t* const x = la;
+        la = lb;
+        lb = x;
+        __syncthreads();
+    }
+    if (t == 0) {
+        a.out[0] = nc;
+        a.out[1] = (uint32_t)swap;
+        a.out[2] = err;
+    }
+}
+
 __global__ void k_match_unmatched(uint32_t n, const uint32_t* __restrict__ vcmap, uint32_t* __restrict__ flag)
 {
     const uint32_t i = blockIdx.x * BLOCK + threadIdx.x;
@@ -1929,6 +2104,24 @@ static uint32_t match_rounds(Ctx& c, const DGraph& g, int level, const uint32_t*
     int swap = 1, idle = 0;
     for (uint32_t round = 0; len > 0; round++) {
         MI_CHECK(round <= 2ull * n + 4, ST_INTERNAL, "matching rounds did not end");
+        if (len <= MATCH_ONE_WG) {
+            const MatchTail a{len,     nc,      (uint32_t)(2ull * n + 4 - round), swap, idle, level,
+                              g.R(),   g.Cc(),  g.W(),         pos,           la.get(),      lb.get(),
+                              hn,      vcmap,   B.est.get(),   B.first.get(), B.flag.get(),  B.cnt.get()};
+            // (a lane or a few per short row; long rows by whole wavefronts)
+            if (g.m >= 32ull * n)
+                k_match_tail<WAVE><<<1, MATCH_BLOCK, 0, c.stream>>>(a);
+            else
+                k_match_tail<8><<<1, MATCH_BLOCK, 0, c.stream>>>(a);
+            MI_HIP(hipGetLastError());
+            uint32_t h[3] = {0, 0, 0};
+            read_words(c, B.cnt.get(), h, 12);
+            MI_CHECK(h[2] != 2, ST_INTERNAL, "matching rounds did not end");
+            MI_CHECK(h[2] != 1, ST_ARG, "matching: only self-loops left");
+            nc = h[0];
+            swap = (int)h[1];
+            break;
+        }
         const uint32_t pairs = match_round(c, B, len, la.get(), hn, pos, swap, nc, vcmap);
         nc += pairs;
         // the next list: unmatched vertices with an unmatched neighbour, in order

@@ -124,3 +124,20 @@ def test_dropin_match(tmp_path, fm):
     else:
         o = oracle.partition_graph(rp, col, None, 33, 33, variant=1)
         assert [l["number-vertices"] for l in t["coarse-levels"]] == [int(x) for x in o["levels_n"]][::-1]
+
+
+@pytest.mark.parametrize("n", [2, 63, 1024, 1025, 4095, 4096, 4097, 6000])
+def test_match_list_ends_in_one_workgroup(mt, n):
+    """Lists of at most 4096 slots run their rounds in one workgroup (1024
+    slots at a time), longer ones until they are that short."""
+    rng = np.random.default_rng(n)
+    k = np.arange(n - 1)
+    for extra, wmax in ((0, 1), (n, 3), (20 * n, 9)):  # (the last: rows by whole wavefronts)
+        u, v = np.concatenate([k, rng.integers(0, n, extra)]), np.concatenate([k + 1, rng.integers(0, n, extra)])
+        rp, col, w = graphs.from_edges(n, u, v, rng.integers(1, wmax + 1, len(u)), lcc=False)
+        g = mt.graph(rp, col, w)
+        for level in (1, 2):
+            vc, nc, _, _ = g.hec_level(level, 7)
+            ovc, onc, _ = oracle.coarsen_match(level, rp, col, w, 7)
+            assert nc == onc and np.array_equal(vc, ovc)
+        g.close()
