@@ -424,6 +424,187 @@ __global__ void k_map_assign2(uint32_t n, const uint32_t* __restrict__ pos, cons
     }
 }
 
+// The whole closed form of a level of at most MAP_LDS vertices in one
+// workgroup, its arrays in LDS: the phases of the kernels above, barriers where
+// those end.  By launches a level costs some sixteen of them, about 90 us
+// whatever its size (the maps of all levels of the 2d grid 64^2 0.29 ms by
+// launches and 0.12 ms so, of the random geometric graph of 100,003 vertices,
+// whose three largest are above the line, 0.85 and 0.55 ms).
+// nonact: heavy-neighbour children not yet known to be passive.
+// out: ids of pass 1, of pass 2, vertices left unresolved, the largest id.
+constexpr uint32_t MAP_LDS = 4096;
+constexpr int MAP_BLOCK = 1024;
+__global__ void __launch_bounds__(MAP_BLOCK) k_map_lds(uint32_t n, const uint32_t* __restrict__ vperm_g,
+                                                       const uint32_t* __restrict__ pos_g,
+                                                       const uint32_t* __restrict__ hn_g,
+                                                       const uint8_t* __restrict__ pre, uint32_t nc0,
+                                                       uint32_t* __restrict__ vcmap_g, uint32_t* __restrict__ out)
+{
+    __shared__ uint32_t first[MAP_LDS], kids[MAP_LDS], vc[MAP_LDS];
+    __shared__ uint16_t vperm[MAP_LDS], pos[MAP_LDS], hn[MAP_LDS], id[MAP_LDS];
+    __shared__ uint8_t fl[MAP_LDS], claimed[MAP_LDS], held[MAP_LDS];
+    __shared__ uint32_t wsum[2][MAP_BLOCK / WAVE], left, largest;
+    const uint32_t t = threadIdx.x, lane = t & (WAVE - 1), wv = t / WAVE;
+    const auto each = [&](auto&& f) {
+        for (uint32_t u = t; u < n; u += MAP_BLOCK) f(u);
+    };
+    // id[i] = number of flags before i; returns the number of all
+    int turn = 0;
+    const auto number = [&](auto&& flag) {
+        uint32_t sum = 0;
+        for (uint32_t i0 = 0; i0 < n; i0 += MAP_BLOCK) {
+            const uint32_t i = i0 + t;
+            const bool f = i < n && flag(i);
+            const unsigned long long b = __ballot(f);
+            if (lane == 0) wsum[turn][wv] = (uint32_t)__popcll(b);
+            __syncthreads();
+            uint32_t before = 0, all = 0;
+            for (uint32_t j = 0; j < MAP_BLOCK / WAVE; j++) {
+                before += j < wv ? wsum[turn][j] : 0u;
+                all += wsum[turn][j];
+            }
+            turn ^= 1;  // (one barrier per tile: the next one's counts go elsewhere)
+            if (i < n) id[i] = (uint16_t)(sum + before + (uint32_t)__popcll(b & ((1ull << lane) - 1ull)));
+            sum += all;
+        }
+        return sum;
+    };
+    each([&](uint32_t u) {
+        vperm[u] = (uint16_t)vperm_g[u];
+        pos[u] = (uint16_t)pos_g[u];
+        hn[u] = (uint16_t)hn_g[u];
+        first[u] = INF;
+        kids[u] = 0;
+        claimed[u] = 0;
+        held[u] = pre && pre[u] ? 1 : 0;
+        vc[u] = held[u] ? vcmap_g[u] : INF;
+    });
+    if (t == 0) largest = 0;
+    __syncthreads();
+    // ---- pass 1
+    each([&](uint32_t u) {
+        const uint32_t v = hn[u];
+        const bool e = !held[u] && pos[u] >= pos[v];
+        fl[u] = e ? FL_E : 0;
+        if (e && v != u) atomicMin(&first[v], (uint32_t)pos[u]);
+    });
+    __syncthreads();
+    const auto creates1 = [&](uint32_t i) {
+        const uint32_t u = vperm[i], v = hn[u];
+        return (fl[u] & FL_E) && (v == u || (!(fl[v] & FL_E) && !held[v] && first[v] == i));
+    };
+    const uint32_t nc1 = number(creates1);
+    __syncthreads();
+    // (the flag's own bit takes no part in creates1)
+    each([&](uint32_t i) {
+        const uint32_t u = vperm[i];
+        if (creates1(i)) fl[u] = FL_E | FL_CR;
+    });
+    __syncthreads();
+    each([&](uint32_t u) {
+        if (fl[u] & FL_CR) {
+            const uint32_t c = nc0 + id[pos[u]];
+            vc[u] = c;
+            if (hn[u] != u) vc[hn[u]] = c;
+        } else if (fl[u] & FL_E) {
+            // follow hn while it stays inside E; positions strictly decrease
+            uint32_t x = u, root = u, c = INF;
+            for (uint32_t step = 0; step <= n; step++) {
+                if (fl[x] & FL_CR) {
+                    root = x;
+                    break;
+                }
+                const uint32_t v = hn[x];
+                if (fl[v] & FL_E) {
+                    x = v;
+                } else if (held[v]) {
+                    c = vc[v];  // a prefilled id: never written here
+                    break;
+                } else {
+                    root = vperm[first[v]];
+                    break;
+                }
+            }
+            vc[u] = c != INF ? c : nc0 + id[pos[root]];
+        }
+    });
+    __syncthreads();
+    // ---- pass 2
+    each([&](uint32_t u) {
+        if (vc[u] == INF) fl[u] |= FL_R;
+        first[u] = INF;
+    });
+    __syncthreads();
+    each([&](uint32_t u) {
+        if ((fl[u] & FL_R) && (fl[hn[u]] & FL_R)) atomicAdd(&kids[hn[u]], 1u);
+    });
+    uint32_t open = 1;
+    for (uint32_t round = 0; open && round <= n + 8; round++) {
+        __syncthreads();
+        if (t == 0) left = 0;
+        __syncthreads();
+        each([&](uint32_t u) {
+            const uint8_t f = fl[u];
+            if (!(f & FL_R) || (f & (FL_ACT | FL_NACT))) return;
+            if (claimed[u])
+                fl[u] = f | FL_NACT;
+            else if (kids[u] == 0)
+                fl[u] = f | FL_ACT;
+            else
+                left = 1;
+        });
+        __syncthreads();
+        open = left;
+        each([&](uint32_t u) {
+            const uint8_t f = fl[u];
+            if (!(f & FL_R) || !(f & (FL_ACT | FL_NACT)) || (f & FL_PROP)) return;
+            const uint32_t v = hn[u];
+            if (fl[v] & FL_R) {
+                if (f & FL_ACT)
+                    claimed[v] = 1;
+                else
+                    atomicSub(&kids[v], 1u);
+            }
+            fl[u] = f | FL_PROP;
+        });
+    }
+    __syncthreads();
+    each([&](uint32_t u) {
+        const uint8_t f = fl[u];
+        if ((f & FL_R) && (f & FL_ACT) && (fl[hn[u]] & FL_R)) atomicMin(&first[hn[u]], (uint32_t)pos[u]);
+    });
+    __syncthreads();
+    const uint32_t nc2 = number([&](uint32_t i) {
+        const uint32_t u = vperm[i];
+        const uint8_t f = fl[u];
+        return (f & FL_R) && (f & FL_ACT) && (fl[hn[u]] & FL_R) && first[hn[u]] == i;
+    });
+    __syncthreads();
+    uint32_t most = 0;
+    if (!open) {
+        each([&](uint32_t u) {
+            uint32_t c = vc[u];
+            if (fl[u] & FL_R) {
+                // (a vertex that joins one with an id: that one is not in R)
+                if ((fl[u] & FL_ACT) && !(fl[hn[u]] & FL_R))
+                    c = vc[hn[u]];
+                else
+                    c = nc0 + nc1 + id[first[(fl[u] & FL_ACT) ? hn[u] : u]];
+            }
+            vcmap_g[u] = c;
+            most = c > most ? c : most;
+        });
+    }
+    atomicMax(&largest, most);
+    __syncthreads();
+    if (t == 0) {
+        out[0] = nc1;
+        out[1] = nc2;
+        out[2] = open;
+        out[3] = largest;
+    }
+}
+
 // max over vcmap, so the host can verify every vertex got a cluster id < nc
 // (fixed grid, one atomic per workgroup)
 __global__ void __launch_bounds__(BLOCK) k_max_u32(const uint32_t* __restrict__ a, uint32_t n,
@@ -2383,6 +2564,20 @@ static uint32_t gosh_map(Ctx& c, const DGraph& g, uint32_t* vcmap, HecTimes* t)
 static uint32_t map_closed_form(Ctx& c, uint32_t n, const uint32_t* vperm, const uint32_t* pos, const uint32_t* hn,
                                 uint32_t* vcmap, const uint8_t* pre, uint32_t nc0)
 {
+    const auto ended = [nc0](const uint32_t (&tot)[4]) {
+        MI_CHECK(tot[2] == 0, ST_INTERNAL, "map construction did not converge");
+        MI_CHECK(nc0 + tot[0] + tot[1] >= 1 && tot[3] < nc0 + tot[0] + tot[1], ST_INTERNAL,
+                 "map construction left a vertex without a cluster id");
+        return nc0 + tot[0] + tot[1];
+    };
+    uint32_t tot[4] = {0, 0, 0, 0};
+    if (n <= MAP_LDS) {
+        DBuf<uint32_t> out(&c.pool, 4);
+        k_map_lds<<<1, MAP_BLOCK, 0, c.stream>>>(n, vperm, pos, hn, pre, nc0, vcmap, out.get());
+        MI_HIP(hipGetLastError());
+        read_words(c, out.get(), tot, 16);
+        return ended(tot);
+    }
     DBuf<uint8_t> fl(&c.pool, n);
     DBuf<uint32_t> minpos(&c.pool, n), id(&c.pool, n);
     // one zero fill for the four totals and pass 2's three counters
@@ -2446,13 +2641,8 @@ static uint32_t map_closed_form(Ctx& c, uint32_t n, const uint32_t* vperm, const
     MI_HIP(hipGetLastError());
     k_max_u32<<<red_grid(n), BLOCK, 0, c.stream>>>(vcmap, n, totals + 3);
     MI_HIP(hipGetLastError());
-    uint32_t tot[4] = {0, 0, 0, 0};
     read_words(c, totals, tot, 16);
-    MI_CHECK(tot[2] == 0, ST_INTERNAL, "map construction did not converge");
-    MI_CHECK(nc0 + tot[0] + tot[1] >= 1 && tot[3] < nc0 + tot[0] + tot[1], ST_INTERNAL,
-             "map construction left a vertex without a cluster id");
-    return nc0 + tot[0] + tot[1];
-
+    return ended(tot);
 }
 
 uint32_t hec_map(Ctx& c, const DGraph& g, const uint32_t* roc, int level, uint64_t seed, uint32_t* vcmap,

@@ -6,6 +6,7 @@ hierarchy's own levels against the oracle: test_gpu_parity.py."""
 import numpy as np
 import pytest
 
+import oracle
 from ipdps_2021_graph_coarsening_amd import graphs
 
 pytestmark = pytest.mark.gpu
@@ -33,3 +34,23 @@ def test_levels_one_by_one(ctx, n, variant):
         g.close()
     finally:
         ctx.set_coarsening(0)
+
+
+@pytest.mark.parametrize("n", [1, 2, 65, 1023, 1024, 1025, 4095, 4096, 4097])
+def test_map_in_one_workgroup(ctx, n):
+    """Maps of at most 4096 vertices are made in one workgroup's LDS: against
+    the oracle, with isolated vertices too (prefilled maps: test_gpu_gosh2.py)."""
+    rng = np.random.default_rng(n)
+    k = np.arange(n - 1)
+    for chain in (True, False):
+        u, v = rng.integers(0, n, n), rng.integers(0, n, n)
+        if chain:
+            u, v = np.concatenate([k, u]), np.concatenate([k + 1, v])
+        rp, col, w = graphs.from_edges(n, u, v, rng.integers(1, 4, len(u)), lcc=False)
+        for level in (1, 2):
+            g = ctx.graph(rp, col, w)
+            vc, nc, vperm, hn = g.hec_level(level, 11)
+            ovc, onc, ovperm, ohn = oracle.coarsen_hec(level, rp, col, w, 11)
+            assert np.array_equal(vperm, ovperm) and np.array_equal(hn, ohn)
+            assert nc == onc and np.array_equal(vc, ovc)
+            g.close()
