@@ -959,18 +959,26 @@ static void keys_to_csr(Ctx& c, DBuf<K>& keys, DBuf<uint32_t>& vals, uint64_t m,
     out.col_sorted = !first_order;  // rows by key: columns ascending
 }
 
-// the largest weight of a level (one atomic per wavefront)
-__global__ void k_wmax(uint64_t m, const uint32_t* __restrict__ w, uint32_t* __restrict__ out)
+// the largest weight of a level
+// (one atomic per workgroup, and few of those: 16,384 wavefronts' atomics on
+// the same word took 190 us whatever the level's size, 18 us so)
+__global__ void __launch_bounds__(BLOCK) k_wmax(uint64_t m, const uint32_t* __restrict__ w,
+                                                uint32_t* __restrict__ out)
 {
+    __shared__ uint32_t lds[BLOCK / WAVE];
     uint32_t v = 0;
-    for (uint64_t e = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; e < m; e += (uint64_t)gridDim.x * BLOCK)
-        v = w[e] > v ? w[e] : v;
+    const uint64_t step = (uint64_t)gridDim.x * BLOCK;
+    uint64_t e = (uint64_t)blockIdx.x * BLOCK + threadIdx.x;
+    for (; e + 7 * step < m; e += 8 * step) {
+        uint32_t x[8];
 #pragma unroll
-    for (int o = WAVE / 2; o > 0; o >>= 1) {
-        const uint32_t x = __shfl_xor(v, o, WAVE);
-        v = x > v ? x : v;
+        for (int k = 0; k < 8; k++) x[k] = w[e + k * step];
+#pragma unroll
+        for (int k = 0; k < 8; k++) v = x[k] > v ? x[k] : v;
     }
-    if ((threadIdx.x & (WAVE - 1)) == 0 && v) atomicMax(out, v);
+    for (; e < m; e += step) v = w[e] > v ? w[e] : v;
+    v = block_max_u32(v, lds);
+    if (threadIdx.x == 0 && v) atomicMax(out, v);
 }
 
 // The sort moves (key, weight) pairs, or keys alone: for unit weights, and
@@ -986,7 +994,7 @@ static void build_coarse_impl(Ctx& c, const DGraph& g, const uint32_t* roc, cons
     if (sizeof(K) == 8 && g.W() && !c.hashmap && m) {
         DBuf<uint32_t> mx(&c.pool, 1);
         fill_u32(c, mx.get(), 1, 0u);
-        k_wmax<<<(unsigned)std::min<uint64_t>(ceil_div(m, BLOCK), 4096), BLOCK, 0, c.stream>>>(m, g.W(), mx.get());
+        k_wmax<<<(unsigned)std::min<uint64_t>(ceil_div(m, 8 * BLOCK), 1024), BLOCK, 0, c.stream>>>(m, g.W(), mx.get());
         MI_HIP(hipGetLastError());
         uint32_t wmax = 0;
         read_words(c, mx.get(), &wmax, 4);
