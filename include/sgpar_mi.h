@@ -45,7 +45,10 @@ typedef struct mi_hier mi_hier;
 /* Mirrors config_t, sgpar.h:186-193 (same fields, same order). */
 typedef struct {
     int coarsening_alg;   /* ignored on this path, as in the reference's Kokkos branch */
-    int refine_alg;       /* 0: Laplacian, 1: normalised Laplacian (normLap) */
+    int refine_alg;       /* 0: Laplacian, 1: normalised Laplacian (normLap):
+                             the loop takes the constant vector out once, so
+                             where it stops depends on the last bits of the
+                             sums; their order is the same for every call */
     int local_search_alg; /* 0 only (the reference returns before local search); FM refinement is
                              the context's mi_ctx_set_refinement, as it is a build flag there */
     int num_iter;         /* trials; the library runs one trial per call */
@@ -109,9 +112,10 @@ int mi_ctx_set_precision(mi_ctx* ctx, int mixed, uint32_t min_entries);
    (default 131072, at most 262144; 0: none) run their whole FP64 power
    iteration in one workgroup, consecutive such levels in one launch, chunk
    iterations per launch at most (0: 8192),
-   instead of two kernel launches per iteration.  Same stop rule and
-   result bookkeeping; the sums are added in another order.  No counterpart
-   in the reference. */
+   instead of launches per iteration.  Same stop rule and
+   result bookkeeping; the sums are added in another order.  Under the
+   normalised Laplacian: levels of at most 16384 vertices and max_entries
+   entries, a launch each.  No counterpart in the reference. */
 int mi_ctx_set_small_levels(mi_ctx* ctx, uint32_t max_entries, uint32_t chunk);
 /* enable != 0 (the default): a level above the finest with at least
    min_vertices vertices (0: 65536) whose power step gathers x from global

@@ -248,8 +248,9 @@ class Context:
         self.check(self._L.mi_ctx_set_builder(self.h, builder), "mi_ctx_set_builder")
 
     def set_small_levels(self, max_entries: int = 1 << 17, chunk: int = 0) -> None:
-        """Levels of <= 7168 vertices and <= max_entries entries iterate in one
-        workgroup (0: never), at most chunk iterations per launch (0: 8192)."""
+        """Levels of <= 7168 vertices (normalised Laplacian: 16384) and <=
+        max_entries entries iterate in one workgroup (0: never), at most chunk
+        iterations per launch (0: 8192)."""
         self.check(self._L.mi_ctx_set_small_levels(self.h, max_entries, chunk), "mi_ctx_set_small_levels")
 
     def set_precision(self, mixed: bool, min_entries: int = 0) -> None:

@@ -384,7 +384,7 @@ DBuf<double> fiedler_levels(Ctx& c, const std::vector<DLevel>& lv, int from, DBu
         PowerStats ps;
         // consecutive small levels: one launch
         int e = l;
-        while (e >= 0 && !local[e] && small_level(c, lv[e].g, mixed_at(e))) e--;
+        while (e >= 0 && !local[e] && small_level(c, lv[e].g, mixed_at(e), normLap)) e--;
         if (e < l) {
             const int last = e + 1;
             std::vector<SmallChain> chain(1);
@@ -1099,7 +1099,7 @@ void bisect_many(Ctx& c, const std::vector<const DGraph*>& gs, const mi_config* 
         for (; l >= 0; l--) {
             const DGraph& g = H[k][l].g;
             const bool mixed = c.mixed && l > 0 && g.m >= c.mixed_min_m;
-            if (!small_level(c, g, mixed)) break;
+            if (!small_level(c, g, mixed, normLap)) break;
             SmallChainLevel s;
             s.g = &g;
             s.vcmap = l == L - 1 ? nullptr : H[k][l].vcmap.get();

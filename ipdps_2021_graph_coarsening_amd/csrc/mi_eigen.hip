@@ -46,9 +46,11 @@
 // y, and the four sums, reduced per workgroup.  Every sum has a fixed order,
 // so results are bit-identical run to run.
 //
-// Small levels run the whole loop in one workgroup (mi_small.hip), levels
-// without long rows one launch per iteration (mi_rows.hip).  Value
-// type V = float is the mixed-precision form of the two kernels above.
+// Under the plain Laplacian small levels run the whole loop in one workgroup
+// (mi_small.hip) and levels without long rows one launch per iteration
+// (mi_rows.hip).  k_power_small_lds / k_power_small: small levels under the
+// normalised one, with the same range streaming.  Value type V = float is the
+// mixed-precision form of the two kernels above.
 #include "mi_kernels.hpp"
 
 #include <algorithm>
@@ -1329,6 +1331,381 @@ __global__ void __launch_bounds__(BLOCK) k_power_finish(StepArgs A)
     }
 }
 
+// Small levels under the normalised Laplacian (n <= XB, few entries): the whole
+// power iteration in one 1024-thread workgroup, with no kernel boundary between
+// iterations.  That loop takes the constant vector out once, before the first
+// iteration; what rounding leaves of it grows against the rest from then on, so
+// that the iteration at which the loop stops, and with it the partition,
+// depends on the order of every sum.  These forms and the two-kernel step fix
+// that order for normLap; the faster forms of mi_small.hip and mi_rows.hip add
+// in another and are for the plain Laplacian, where the constant is taken out
+// in every iteration (of 140 normalised bisections of meshes 39 changed with
+// the order, by up to 26 % of the cut, of 240 plain ones none).  Every
+// iteration is the two-kernel step above in one place: the stop test on the
+// previous iteration's sums, x = (y - a) s staged in LDS, the ranges of
+// entries streamed by the 16 wavefronts in turn (stream_range, LDS form,
+// one column block), then one thread per row adds its partials, forms y and
+// the four sums, which the workgroup reduces in a fixed order.  The
+// workgroup's own global stores (partials, y) are read back after a
+// workgroup barrier, which orders them within the CU.  A launch runs at
+// most `chunk` iterations and leaves its state (iteration count, the last
+// two dot products, the last sums, a and s) where the next launch resumes
+// it; the launch that reaches the stop leaves the bookkeeping of the
+// two-kernel loop (done flag, iteration count, a and s of the last
+// iteration), so the result is read the same way.
+template <int WF, bool R16>
+__global__ void __launch_bounds__(LBLOCK) k_power_small(StepArgs A, double* buf0, double* buf1, uint32_t chunk)
+{
+    constexpr bool NORMLAP = true;
+    __shared__ double xl[XB];
+    __shared__ double red[4][LNW];
+    const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1), wid = tid / WAVE;
+    const bool lead = tid == 0;
+    if (A.cnt[CT_DONE]) return;
+    const double* part = static_cast<const double*>(A.part);
+    const double* head = static_cast<const double*>(A.head);
+    const double* tail = static_cast<const double*>(A.tail);
+    const uint32_t gb = NORMLAP ? 0u : *A.gbp;
+    uint32_t iter = A.cnt[CT_ITER] + 1u;  // 1-based index of the next iteration
+    double T[4], dot0 = A.scal[SC_DOT], dot1 = A.scal[SC_DOT + 1];
+    double last_a = A.scal[SC_A], last_s = A.scal[SC_S];
+#pragma unroll
+    for (int k = 0; k < 4; k++) T[k] = A.fcur[k];  // (fcur[0..4) holds the sums between launches)
+    for (uint32_t it = 0; it < chunk; it++, iter++) {
+        double a = 0.0, s = 1.0;
+        if (iter >= 2) {
+            // the stop test of iteration iter - 1 (iteration_start's formulas)
+            const double an = T[0] * A.c * A.c;
+            const double nrm2 = T[1] - 2.0 * an * T[0] + an * an * (double)A.n;
+            const double sn = 1 / sqrt(nrm2);
+            const double dot = (T[2] - an * T[3]) * sn;
+            const unsigned long long itn = iter - 1;
+            const double lastd = (iter & 1u) ? dot1 : dot0;
+            const bool go_on = (fabs(dot - lastd) > A.tol) && (itn < A.iter_max);
+            if ((iter - 1) & 1u)
+                dot1 = dot;
+            else
+                dot0 = dot;
+            if (!go_on) {
+                if (lead) {
+                    A.scal[SC_DOT] = dot0;
+                    A.scal[SC_DOT + 1] = dot1;
+                    A.scal[SC_A] = last_a;
+                    A.scal[SC_S] = last_s;
+                    A.cnt[CT_ITER] = iter - 1;
+                    A.cnt[CT_DONE] = 1u;
+                    A.cnt[CT_MAXR] = itn >= A.iter_max ? 1u : 0u;
+                    *A.niter = itn;
+                }
+                return;
+            }
+            a = an;
+            s = sn;
+        }
+        last_a = a;
+        last_s = s;
+        const double* yp = ((iter - 1) & 1u) ? buf1 : buf0;
+        double* yn = (iter & 1u) ? buf1 : buf0;
+        for (uint32_t i = tid; i < A.n; i += LBLOCK) xl[i] = (yp[i] - a) * s;
+        __syncthreads();
+        {
+            const RangeSeq S{0u, A.m, 0u, A.B.pw, (uint32_t)LNW, A.nwaves, nullptr};
+            PassQueue<1> Q;
+            pq_init<WF, true, R16>(A, Q, S, wid);
+            for (uint32_t wv = wid; wv < A.nwaves; wv += LNW) {
+                uint32_t E0, E1;
+                S.bounds(wv, E0, E1);
+                const uint32_t nrow = (wv + 1 < A.nwaves) ? (A.wmeta[wv + 1] & ~HEADF) : RINF;
+                stream_range<WF, true, R16, double>(A, wv, E0, E1, nrow, a, s, xl, Q, S);
+            }
+        }
+        __syncthreads();
+        double S[4] = {0.0, 0.0, 0.0, 0.0};
+        for (uint32_t r = tid; r < A.n; r += LBLOCK) {
+            const double v = row_total<1, false>(A, r, 1u, part, head, tail);
+            const double xr = xl[r];
+            const double y = shifted<NORMLAP>(A, v, xr, A.wdeg ? A.wdeg[r] : 0u, gb);
+            yn[r] = y;
+            S[0] += NORMLAP ? 0.0 : y;
+            S[1] += y * y;
+            S[2] += xr * y;
+            S[3] += xr;
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const double w = wave_sum(S[k]);
+            if (lane == 0) red[k][wid] = w;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            double t = 0.0;
+#pragma unroll
+            for (int j = 0; j < LNW; j++) t += red[k][j];
+            T[k] = t;
+        }
+        __syncthreads();  // red and xl are rewritten by the next iteration
+    }
+    if (lead) {
+        A.cnt[CT_ITER] = iter - 1;
+        A.scal[SC_DOT] = dot0;
+        A.scal[SC_DOT + 1] = dot1;
+        A.scal[SC_A] = last_a;
+        A.scal[SC_S] = last_s;
+#pragma unroll
+        for (int k = 0; k < 4; k++) A.fcur[k] = T[k];
+    }
+}
+
+// The same loop with every vector in LDS, for levels where x, y, the row
+// partials and the range partials fit there together (2 n + 2 ranges <=
+// SMALL_LDS doubles, the row partials sharing y's space; rows <= 8 per
+// thread, instances for 4 and 8): only the matrix is read from
+// global memory (and stays in the caches), and each thread keeps its rows'
+// range indices and weighted degrees in registers for the whole loop.
+// stream_range writes the partials through generic pointers into LDS.  Each
+// thread stages x and forms y for the same indices (its rows), so x and y
+// need no barrier between those two steps.  A launch starts from y in
+// global memory; when its chunk ends it leaves y of its last iteration in
+// that iteration's output buffer and x of that iteration in the other one.
+// At the stop, x of the last iteration goes to `out`.
+//
+// The first launch also prepares the start vector, as the two-kernel loop's
+// setup kernels do (eigensolve_kokkos.h:118-150): u = start (or
+// start[vcmap[i]], the prolongation from the coarser level), orthogonalised
+// against 1n (normLap 0: u -= (u . 1n) 1n; normLap 1: u -= (sum u D 1n /
+// sum 1n D 1n) 1n) and normalised, with the sums taken in this workgroup.
+constexpr uint32_t SMALL_LDS = 18432;  // doubles (144 KiB)
+constexpr uint32_t SMALL_RPT = 8;      // rows per thread at most (instances for 4 and 8)
+
+// Sum of v over the workgroup, in every thread (a fixed order); red[0] is
+// reused, behind barriers on both sides.
+__device__ __forceinline__ double small_block_sum(double v, double (*red)[LNW])
+{
+    const uint32_t lane = threadIdx.x & (WAVE - 1), wid = threadIdx.x / WAVE;
+    v = wave_sum(v);
+    __syncthreads();
+    if (lane == 0) red[0][wid] = v;
+    __syncthreads();
+    double t = 0.0;
+#pragma unroll
+    for (int j = 0; j < LNW; j++) t += red[0][j];
+    return t;
+}
+
+template <int WF, bool R16, bool NORMLAP, uint32_t RPT>
+__device__ __forceinline__ void small_loop(const StepArgs& A, double* buf0, double* buf1, uint32_t chunk,
+                                           const double* start, const uint32_t* vcmap, double* out, double* sm,
+                                           double (*red)[LNW])
+{
+    const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1), wid = tid / WAVE;
+    const bool lead = tid == 0;
+    if (A.cnt[CT_DONE]) return;
+    const uint32_t n = A.n, nw = A.nwaves;
+    double* xl = sm;
+    double* yl = sm + n;
+    double* pl = yl;  // (y of the previous iteration is dead once x is staged)
+    double* hl = sm + 2 * n;
+    double* tl = hl + nw;
+    StepArgs B = A;  // the partials go to LDS
+    B.part = pl;
+    B.head = hl;
+    B.tail = tl;
+    const uint32_t gb = NORMLAP ? 0u : *A.gbp;
+    // this thread's rows: range of the first and last entry, weighted degree
+    uint32_t w0[RPT], w1[RPT], wd[RPT];
+    bool has[RPT];
+#pragma unroll
+    for (uint32_t k = 0; k < RPT; k++) {
+        const uint32_t r = tid + k * LBLOCK;
+        has[k] = false;
+        w0[k] = w1[k] = wd[k] = 0;
+        if (r < n) {
+            const uint32_t s0 = A.rowptr[r], s1 = A.rowptr[r + 1];
+            has[k] = s0 != s1;
+            if (has[k]) {
+                w0[k] = s0 >> A.B.pws;
+                w1[k] = (s1 - 1) >> A.B.pws;
+            }
+            wd[k] = A.wdeg ? A.wdeg[r] : 0u;
+        }
+    }
+    uint32_t iter = A.cnt[CT_ITER] + 1u;  // 1-based index of the next iteration
+    double T[4], dot0 = A.scal[SC_DOT], dot1 = A.scal[SC_DOT + 1];
+#pragma unroll
+    for (int k = 0; k < 4; k++) T[k] = A.fcur[k];  // (fcur[0..4) holds the sums between launches)
+    if (iter == 1) {
+        // the start vector, orthogonalised and normalised
+        const double c = A.c;
+        double p0 = 0.0, p1 = 0.0;
+        for (uint32_t i = tid; i < n; i += LBLOCK) {
+            const double u = vcmap ? start[vcmap[i]] : start[i];
+            yl[i] = u;
+            if (!NORMLAP) {
+                p0 += u * c;
+            } else {
+                const double d = (double)A.wdeg[i];
+                p0 += u * d * c;
+                p1 += c * d * c;
+            }
+        }
+        const double num = small_block_sum(p0, red);
+        const double shift = NORMLAP ? num * c / small_block_sum(p1, red) : num * c;
+        double q = 0.0;
+        for (uint32_t i = tid; i < n; i += LBLOCK) {
+            const double u = yl[i] - shift;
+            yl[i] = u;
+            q += u * u;
+        }
+        const double inv = 1 / sqrt(small_block_sum(q, red));
+        for (uint32_t i = tid; i < n; i += LBLOCK) yl[i] = yl[i] * inv;
+    } else {
+        const double* y0 = ((iter - 1) & 1u) ? buf1 : buf0;
+        for (uint32_t i = tid; i < n; i += LBLOCK) yl[i] = y0[i];
+    }
+    for (uint32_t it = 0; it < chunk; it++, iter++) {
+        double a = 0.0, s = 1.0;
+        if (iter >= 2) {
+            const double an = T[0] * A.c * A.c;
+            const double nrm2 = T[1] - 2.0 * an * T[0] + an * an * (double)n;
+            const double sn = 1 / sqrt(nrm2);
+            const double dot = (T[2] - an * T[3]) * sn;
+            const unsigned long long itn = iter - 1;
+            const double lastd = (iter & 1u) ? dot1 : dot0;
+            const bool go_on = (fabs(dot - lastd) > A.tol) && (itn < A.iter_max);
+            if ((iter - 1) & 1u)
+                dot1 = dot;
+            else
+                dot0 = dot;
+            if (!go_on) {
+                // x of iteration itn: still in LDS, or where the previous
+                // launch left it when this one ran none
+                const double* res = ((itn - 1) & 1u) ? buf1 : buf0;
+                for (uint32_t i = tid; i < n; i += LBLOCK) out[i] = it > 0 ? xl[i] : res[i];
+                if (lead) {
+                    A.cnt[CT_DONE] = 1u;
+                    A.cnt[CT_MAXR] = itn >= A.iter_max ? 1u : 0u;
+                    *A.niter = itn;
+                }
+                return;
+            }
+            a = an;
+            s = sn;
+        }
+        // (every read of x by the previous iteration's gathers ended before
+        // its final barrier)
+        for (uint32_t i = tid; i < n; i += LBLOCK) xl[i] = (yl[i] - a) * s;
+        __syncthreads();
+        {
+            const RangeSeq S{0u, A.m, 0u, A.B.pw, (uint32_t)LNW, nw, nullptr};
+            PassQueue<1> Q;
+            pq_init<WF, true, R16>(B, Q, S, wid);
+            for (uint32_t wv = wid; wv < nw; wv += LNW) {
+                uint32_t E0, E1;
+                S.bounds(wv, E0, E1);
+                const uint32_t nrow = (wv + 1 < nw) ? (A.wmeta[wv + 1] & ~HEADF) : RINF;
+                stream_range<WF, true, R16, double>(B, wv, E0, E1, nrow, a, s, xl, Q, S);
+            }
+        }
+        __syncthreads();
+        double S[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (uint32_t k = 0; k < RPT; k++) {
+            const uint32_t r = tid + k * LBLOCK;
+            if (r < n) {
+                // row_total's order: the first partial, then the heads
+                double v = 0.0;
+                if (has[k]) {
+                    v = w0[k] == w1[k] ? pl[r] : tl[w0[k]];
+                    for (uint32_t q = w0[k] + 1; q <= w1[k]; q++) v += hl[q];
+                }
+                const double xr = xl[r];
+                const double y = shifted<NORMLAP>(A, v, xr, wd[k], gb);
+                yl[r] = y;
+                S[0] += NORMLAP ? 0.0 : y;
+                S[1] += y * y;
+                S[2] += xr * y;
+                S[3] += xr;
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const double w = wave_sum(S[k]);
+            if (lane == 0) red[k][wid] = w;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            double t = 0.0;
+#pragma unroll
+            for (int j = 0; j < LNW; j++) t += red[k][j];
+            T[k] = t;
+        }
+    }
+    // chunk end (iteration iter - 1 >= 1 ran here): its y and x to the
+    // buffers, and the state
+    double* yo = ((iter - 1) & 1u) ? buf1 : buf0;
+    double* xo = ((iter - 1) & 1u) ? buf0 : buf1;
+    for (uint32_t i = tid; i < n; i += LBLOCK) {
+        yo[i] = yl[i];
+        xo[i] = xl[i];
+    }
+    if (lead) {
+        A.cnt[CT_ITER] = iter - 1;
+        A.scal[SC_DOT] = dot0;
+        A.scal[SC_DOT + 1] = dot1;
+#pragma unroll
+        for (int k = 0; k < 4; k++) A.fcur[k] = T[k];
+    }
+}
+
+// Whether a small level's vectors fit in LDS together (k_power_small_lds).
+bool small_lds_fits(uint32_t n, uint32_t nwaves)
+{
+    return n <= SMALL_RPT * LBLOCK && 2ull * n + 2ull * nwaves <= SMALL_LDS;
+}
+
+// One level: its step arguments (with its own loop state), its two work
+// vectors, where its start vector comes from and where its result goes.
+struct SmallJob {
+    StepArgs A;
+    double* b0;
+    double* b1;
+    const double* start;
+    const uint32_t* vcmap;
+    double* out;
+};
+
+// Independent small levels (of different graphs) in one launch, one
+// workgroup each.
+template <bool NORMLAP, uint32_t RPT>
+__global__ void __launch_bounds__(LBLOCK) k_power_small_lds(const SmallJob* __restrict__ jobs, uint32_t chunk)
+{
+    __shared__ double sm[SMALL_LDS];
+    __shared__ double red[4][LNW];
+    const SmallJob& J = jobs[blockIdx.x];
+    const int wf = J.A.wfmt;
+    const bool r16 = J.A.r16 != 0;
+#define MI_SB(WFV, R) small_loop<WFV, R, NORMLAP, RPT>(J.A, J.b0, J.b1, chunk, J.start, J.vcmap, J.out, sm, red)
+    if (wf == W_UNIT) {
+        if (r16)
+            MI_SB(W_UNIT, true);
+        else
+            MI_SB(W_UNIT, false);
+    } else if (wf == W_U16) {
+        if (r16)
+            MI_SB(W_U16, true);
+        else
+            MI_SB(W_U16, false);
+    } else {
+        if (r16)
+            MI_SB(W_U32, true);
+        else
+            MI_SB(W_U32, false);
+    }
+#undef MI_SB
+}
+
 // u = (y - a) * s : the input of the last iteration
 template <class V>
 __global__ void k_materialize(uint32_t n, const V* __restrict__ y, double* __restrict__ u, const double* scal)
@@ -1836,7 +2213,7 @@ LevelStep level_step(Ctx& c, const DGraph& g, const LevelPlan& p, const uint32_t
 void launch_step(Ctx& c, int normLap, const LevelStep& L)
 {
     if (L.by_rows) {
-        launch_rows(c, normLap, L.f32, L.rows);
+        launch_rows(c, L.f32, L.rows);  // (plan_level: never for normLap)
         return;
     }
     const StepArgs& A = L.stream;
@@ -1872,7 +2249,7 @@ static uint32_t column_blocks(uint32_t n, uint32_t m)
     return ncb;
 }
 
-void plan_level(Ctx& c, const DGraph& g, LevelPlan& p, bool f32)
+void plan_level(Ctx& c, const DGraph& g, LevelPlan& p, bool f32, int normLap)
 {
     p.f32 = f32;
     const uint32_t n = g.n, m = g.m;
@@ -1883,8 +2260,9 @@ void plan_level(Ctx& c, const DGraph& g, LevelPlan& p, bool f32)
     // more than gathers from the caches instead of LDS (us per iteration,
     // before and now: 3d grid 128^3, 2.1 M vertices 73 and 47; its levels of
     // 628,115 44 and 35, of 183,554 20.5 and 18, of 48,419 15.0 and 12.5, of
-    // 11,686, whose x fits in LDS whole, 15.6 and 9.7).
-    if (ncb <= 1 && plan_rows(c, g, p.rows)) return;
+    // 11,686, whose x fits in LDS whole, 15.6 and 9.7).  Not for normLap,
+    // whose order of sums stays (see k_power_small).
+    if (!normLap && ncb <= 1 && plan_rows(c, g, p.rows)) return;
     p.ncb = ncb;
     p.bw = ncb ? (uint32_t)ceil_div(n, ncb) : 0u;
     for (int q = 0; q <= MAXCB; q++) p.boff[q] = p.bwave[q] = 0;
@@ -2404,13 +2782,42 @@ static void run_steps(Ctx& c, int normLap, const LevelStep (&A)[2], unsigned lon
     }
 }
 
+// The iteration loop of a small level under the normalised Laplacian whose
+// vectors do not fit in LDS: k_power_small in launches of at most
+// c.small_chunk iterations until one reaches the stop.
+static void run_small(Ctx& c, const StepArgs& A, double* b0, double* b1)
+{
+#define MI_SMALL(WF)                                                                          \
+    do {                                                                                      \
+        if (A.r16)                                                                            \
+            k_power_small<WF, true><<<1, LBLOCK, 0, c.stream>>>(A, b0, b1, c.small_chunk);    \
+        else                                                                                  \
+            k_power_small<WF, false><<<1, LBLOCK, 0, c.stream>>>(A, b0, b1, c.small_chunk);   \
+    } while (0)
+    for (unsigned long long launched = 0;; launched += c.small_chunk) {
+        MI_CHECK(launched <= A.iter_max + c.small_chunk, ST_INTERNAL,
+                 "power iteration did not stop at its iteration cap");
+        if (A.wfmt == W_UNIT)
+            MI_SMALL(W_UNIT);
+        else if (A.wfmt == W_U16)
+            MI_SMALL(W_U16);
+        else
+            MI_SMALL(W_U32);
+        MI_HIP(hipGetLastError());
+        uint32_t done = 0;
+        read_words(c, c.cnt + CT_DONE, &done, 4);
+        if (done) break;
+    }
+#undef MI_SMALL
+}
+
 void power_iter(Ctx& c, const DGraph& g, double* d_u, int normLap, double tol, PowerStats* st, double* eig_log,
                 bool mixed)
 {
     const uint32_t n = g.n;
     MI_CHECK(n > 0, ST_ARG, "empty level");
     auto t0 = std::chrono::steady_clock::now();
-    if (small_level(c, g, mixed)) {
+    if (small_level(c, g, mixed, normLap)) {
         std::vector<SmallChain> one(1);
         one[0].lv.resize(1);
         one[0].lv[0].g = &g;
@@ -2428,7 +2835,7 @@ void power_iter(Ctx& c, const DGraph& g, double* d_u, int normLap, double tol, P
     DBuf<double> d0, d1;  // the loop's vectors
     DBuf<float> f0, f1;   // ... in the mixed form
     LevelPlan plan;
-    plan_level(c, g, plan, mixed);
+    plan_level(c, g, plan, mixed, normLap);
     weighted_degree(c, g, plan, wdeg.get(), gb.get());
 
     // vec1 = 1, normalised: every entry is 1/sqrt(n) (n is exact in FP64)
@@ -2497,7 +2904,10 @@ void power_iter(Ctx& c, const DGraph& g, double* d_u, int normLap, double tol, P
         A[k].stream.fprev = plan.fsum.get() + NSUM * MAXF_LDS * (k ^ 1);  // sums of the previous launch
         A[k].stream.fcur = plan.fsum.get() + NSUM * MAXF_LDS * k;
     }
-    run_steps(c, normLap, A, iter_max);
+    if (normLap && !mixed && plan.ncb == 1 && g.m <= c.small_max_m)
+        run_small(c, A[0].stream, static_cast<double*>(buf[0]), static_cast<double*>(buf[1]));
+    else
+        run_steps(c, normLap, A, iter_max);
     MI_HIP(hipStreamSynchronize(c.stream));
     uint32_t flags[2] = {0, 0};
     read_words(c, c.cnt + CT_DONE, flags, 8);
@@ -2518,6 +2928,146 @@ void power_iter(Ctx& c, const DGraph& g, double* d_u, int normLap, double tol, P
         st->iters = done_iters;
         st->max_reached = flags[1] ? 1 : 0;
         st->ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+    }
+}
+
+bool small_lds_level(const Ctx& c, const DGraph& g)
+{
+    if (g.m == 0 || g.m > c.small_max_m || g.n > XB) return false;
+    const uint32_t pw = g.m >= (1u << 22) ? 2 * PASS : PASS;  // plan_level's range size
+    return small_lds_fits(g.n, (uint32_t)ceil_div(g.m, pw));
+}
+
+// A level of k_power_small_lds: start[vcmap[i]] (start[i] when vcmap is null) is
+// its start vector, out its result.
+struct LdsLevel {
+    const DGraph* g;
+    const uint32_t* vcmap;
+    const double* start;
+    double* out;
+    uint64_t iters;  // results
+    int max_reached;
+};
+
+// The power iterations of independent levels, one workgroup each.
+static void solve_lds_levels(Ctx& c, std::vector<LdsLevel>& lv, int normLap, double tol)
+{
+    const size_t J = lv.size();
+    struct Own {
+        LevelPlan plan;
+        DBuf<uint32_t> wdeg, gb;
+        DBuf<double> b0, b1;
+    };
+    std::vector<Own> own(J);
+    // per job: 8 counters, 16 scalars, the iteration count (zero = a fresh loop)
+    DBuf<uint32_t> cnt(&c.pool, 8 * J);
+    DBuf<double> scal(&c.pool, 16 * J);
+    DBuf<unsigned long long> nit(&c.pool, J);
+    MI_HIP(hipMemsetAsync(cnt.get(), 0, 32 * J, c.stream));
+    MI_HIP(hipMemsetAsync(scal.get(), 0, 128 * J, c.stream));
+    MI_HIP(hipMemsetAsync(nit.get(), 0, 8 * J, c.stream));
+    // jobs of at most 4 rows per thread first (their kernel instance keeps
+    // its rows' metadata in fewer registers), then the others
+    std::vector<size_t> order;
+    for (size_t j = 0; j < J; j++)
+        if (lv[j].g->n <= 4u * LBLOCK) order.push_back(j);
+    const size_t J4 = order.size();
+    for (size_t j = 0; j < J; j++)
+        if (lv[j].g->n > 4u * LBLOCK) order.push_back(j);
+    std::vector<SmallJob> host(J);
+    unsigned long long cap = 0;
+    for (size_t k = 0; k < J; k++) {
+        const size_t j = order[k];
+        const DGraph& g = *lv[j].g;
+        Own& o = own[k];
+        plan_level(c, g, o.plan, false, 1);  // (the streaming form)
+        MI_CHECK(o.plan.ncb == 1 && small_lds_fits(g.n, o.plan.nwaves), ST_INTERNAL,
+                 "level does not fit the one-workgroup form");
+        o.wdeg = DBuf<uint32_t>(&c.pool, g.n);
+        o.gb = DBuf<uint32_t>(&c.pool, 1);
+        weighted_degree(c, g, o.plan, o.wdeg.get(), o.gb.get());
+        o.b0 = DBuf<double>(&c.pool, g.n);
+        o.b1 = DBuf<double>(&c.pool, g.n);
+        SmallJob& h = host[k];
+        h.A = make_args(c, g, o.plan, o.wdeg.get(), o.gb.get(), o.b0.get(), o.b1.get(), tol, 0);
+        h.A.cnt = cnt.get() + 8 * k;
+        h.A.scal = scal.get() + 16 * k;
+        h.A.niter = nit.get() + k;
+        h.A.fprev = o.plan.fsum.get();
+        h.A.fcur = o.plan.fsum.get();
+        h.b0 = o.b0.get();
+        h.b1 = o.b1.get();
+        h.start = lv[j].start;
+        h.vcmap = lv[j].vcmap;
+        h.out = lv[j].out;
+        cap = std::max(cap, h.A.iter_max);
+    }
+    DBuf<uint64_t> jobs(&c.pool, (J * sizeof(SmallJob) + 7) / 8);
+    MI_HIP(hipMemcpyAsync(jobs.get(), host.data(), J * sizeof(SmallJob), hipMemcpyHostToDevice, c.stream));
+    const SmallJob* dj = reinterpret_cast<const SmallJob*>(jobs.get());
+    std::vector<uint32_t> hc(8 * J);
+    for (unsigned long long launched = 0;; launched += c.small_chunk) {
+        MI_CHECK(launched <= cap + c.small_chunk, ST_INTERNAL, "power iteration did not stop at its iteration cap");
+        if (J4) {
+            if (normLap)
+                k_power_small_lds<true, 4><<<(unsigned)J4, LBLOCK, 0, c.stream>>>(dj, c.small_chunk);
+            else
+                k_power_small_lds<false, 4><<<(unsigned)J4, LBLOCK, 0, c.stream>>>(dj, c.small_chunk);
+            MI_HIP(hipGetLastError());
+        }
+        if (J > J4) {
+            if (normLap)
+                k_power_small_lds<true, 8><<<(unsigned)(J - J4), LBLOCK, 0, c.stream>>>(dj + J4, c.small_chunk);
+            else
+                k_power_small_lds<false, 8><<<(unsigned)(J - J4), LBLOCK, 0, c.stream>>>(dj + J4, c.small_chunk);
+            MI_HIP(hipGetLastError());
+        }
+        MI_HIP(hipMemcpyAsync(hc.data(), cnt.get(), 32 * J, hipMemcpyDeviceToHost, c.stream));
+        MI_HIP(hipStreamSynchronize(c.stream));
+        bool all = true;
+        for (size_t j = 0; j < J && all; j++) all = hc[8 * j + CT_DONE] != 0;
+        if (all) break;
+    }
+    std::vector<unsigned long long> hn(J);
+    MI_HIP(hipMemcpyAsync(hn.data(), nit.get(), 8 * J, hipMemcpyDeviceToHost, c.stream));
+    MI_HIP(hipStreamSynchronize(c.stream));
+    for (size_t k = 0; k < J; k++) {
+        lv[order[k]].iters = hn[k];
+        lv[order[k]].max_reached = hc[8 * k + CT_MAXR] ? 1 : 0;
+    }
+}
+
+// The levels of the chains, one of each chain per launch.
+void solve_lds_chains(Ctx& c, std::vector<SmallChain>& chains, int normLap, double tol)
+{
+    size_t depth = 0;
+    for (const SmallChain& ch : chains) depth = std::max(depth, ch.lv.size());
+    std::vector<std::vector<DBuf<double>>> between(chains.size());
+    for (size_t d = 0; d < depth; d++) {
+        auto t0 = std::chrono::steady_clock::now();
+        std::vector<LdsLevel> lv;
+        std::vector<size_t> who;
+        for (size_t j = 0; j < chains.size(); j++) {
+            SmallChain& ch = chains[j];
+            if (d >= ch.lv.size()) continue;
+            const SmallChainLevel& l = ch.lv[d];
+            const double* start = d ? between[j].back().get() : ch.start;
+            double* out = ch.out;
+            if (d + 1 < ch.lv.size()) {
+                between[j].emplace_back(&c.pool, l.g->n);
+                out = between[j].back().get();
+            }
+            lv.push_back(LdsLevel{l.g, l.vcmap, start, out, 0, 0});
+            who.push_back(j);
+        }
+        solve_lds_levels(c, lv, normLap, tol);
+        const double ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+        for (size_t i = 0; i < lv.size(); i++) {
+            SmallChainLevel& l = chains[who[i]].lv[d];
+            l.iters = lv[i].iters;
+            l.max_reached = lv[i].max_reached;
+            l.ms = ms;
+        }
     }
 }
 

@@ -191,7 +191,7 @@ bool plan_rows(Ctx& c, const DGraph& g, RowPlan& p);
 // launches of parity 0 and 1 alternate
 RowStep rows_step(Ctx& c, const DGraph& g, const RowPlan& p, const uint32_t* wdeg, const uint32_t* gb,
                   const void* yprev, void* ynew, double tol, int mode, int parity);
-void launch_rows(Ctx& c, int normLap, bool f32, const RowStep& A);
+void launch_rows(Ctx& c, bool f32, const RowStep& A);
 // out = x and the zero that padding reads
 template <class V>
 void pad_copy(Ctx& c, uint32_t n, const double* x, V* out);
@@ -216,7 +216,8 @@ struct LevelPlan {
     uint32_t nblk_f = 0;  // workgroups of the finish kernel
     bool f32 = false;     // FP32 vectors and row partials (mixed precision)
 };
-void plan_level(Ctx& c, const DGraph& g, LevelPlan& p, bool f32 = false);
+// normLap: always the streaming form (see k_power_small in mi_eigen.hip).
+void plan_level(Ctx& c, const DGraph& g, LevelPlan& p, bool f32 = false, int normLap = 0);
 // Mixed precision applies by default to levels above the finest with at
 // least this many stored entries; smaller ones are bound by launch and
 // reduction latency.
@@ -265,10 +266,14 @@ struct SmallChain {
 };
 // Whether power_iter runs level g in one workgroup (so that it can be chained
 // and batched); mixed: the level would run in mixed precision.
-bool small_level(const Ctx& c, const DGraph& g, bool mixed);
-// The FP64 power iterations of independent chains in one launch, one
-// workgroup each: the same results, bit for bit, as power_iter level by level.
+bool small_level(const Ctx& c, const DGraph& g, bool mixed, int normLap);
+// The FP64 power iterations of independent chains, one workgroup each: the
+// same results, bit for bit, as power_iter level by level.  In one launch, or,
+// under the normalised Laplacian, whose order of sums is fixed
+// (k_power_small_lds), a launch per level.
 void solve_small_chains(Ctx& c, std::vector<SmallChain>& chains, int normLap, double tol);
+bool small_lds_level(const Ctx& c, const DGraph& g);
+void solve_lds_chains(Ctx& c, std::vector<SmallChain>& chains, int normLap, double tol);
 // The final eigenvalue log (eigenvalue, min, max) of level g for vector d_u.
 void eigen_log_level(Ctx& c, const DGraph& g, const double* d_u, double* out3);
 // Locality order for the solve of a level.  gather_form_level: the level's

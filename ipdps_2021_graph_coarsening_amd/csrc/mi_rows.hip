@@ -1,6 +1,7 @@
 // mi_rows.hip -- power-iteration step of levels without long rows: one launch
 // per iteration (eigensolve_kokkos.h:102-206, with the vector helpers of
-// :14-58 and the product KokkosSparse::spmv).
+// :14-58 and the product KokkosSparse::spmv), under the plain Laplacian (the
+// normalised one keeps the streaming step's order of sums, see k_power_small).
 //
 // The streaming step (mi_eigen.hip) sums flat ranges of entries, whatever the
 // rows look like, and so takes a second kernel that joins the pieces of rows,
@@ -224,7 +225,7 @@ __device__ __forceinline__ bool iteration_start(const RowStep& A, double& a, dou
         for (int j = 0; j < NW; j++) t += lds[k][j];
         T[k] = t;
     }
-    const double mult = T[0] * A.c;  // dot(v, vec1); 0 for normLap (S1 is not summed)
+    const double mult = T[0] * A.c;  // dot(v, vec1)
     const double an = mult * A.c;    // subtracted from every entry
     const double nrm2 = T[1] - 2.0 * an * T[0] + an * an * (double)A.n;
     const double sn = 1 / sqrt(nrm2);
@@ -295,7 +296,7 @@ __device__ __forceinline__ uint32_t scalar_word(const uint32_t* p)
 
 // One row: y from z = A y_prev (the shifted product of the reference, or A x
 // in mode 2), stored, and its terms of the sums.
-template <bool NORMLAP, class V>
+template <class V>
 __device__ __forceinline__ void emit_row(const RowStep& A, uint32_t r, V z, V yr, uint32_t wd, uint32_t gb, double a,
                                          double s, double (&S)[sums_of<V>])
 {
@@ -305,12 +306,10 @@ __device__ __forceinline__ void emit_row(const RowStep& A, uint32_t r, V z, V yr
     double y;
     if (A.mode == 2)
         y = ax;
-    else if (!NORMLAP)
-        y = fma((double)(uint32_t)(gb - wd), x, ax);
     else
-        y = 0.5 * x + 0.5 * ax * (1.0 / (double)wd);
+        y = fma((double)(uint32_t)(gb - wd), x, ax);
     static_cast<V*>(A.ynew)[r] = (V)y;
-    if (!NORMLAP) S[0] += y;
+    S[0] += y;
     S[1] = fma(y, y, S[1]);
     S[2] = fma(x, y, S[2]);
     if (sums_of<V> == 4) S[sums_of<V> - 1] = fma(x, x, S[sums_of<V> - 1]);
@@ -338,14 +337,14 @@ __device__ __forceinline__ void leave_sums(const RowStep& A, const double (&S)[N
 // and 11.4.
 // Wavefront k of the logical grid takes the slices span[k] ..
 // span[k + 1].  The first slice is summed before a and s are known.
-template <int WF, bool NORMLAP, class V>
+template <int WF, class V>
 __global__ void __launch_bounds__(BLOCK) k_power_rows(RowStep A)
 {
     const V* yp = static_cast<const V*>(A.yprev);
     const uint32_t lane = threadIdx.x & (WAVE - 1), k = uniform(logical_block() * NW + threadIdx.x / WAVE);
     uint32_t sl = scalar_word(A.span + k);
     const uint32_t end = scalar_word(A.span + k + 1);
-    const uint32_t gb = (NORMLAP || A.mode == 2) ? 0u : *A.gbp;
+    const uint32_t gb = A.mode == 2 ? 0u : *A.gbp;
     V z = 0, yr = 0;
     uint32_t row = INF, wd = 0;
     auto slice = [&]() {
@@ -375,7 +374,7 @@ __global__ void __launch_bounds__(BLOCK) k_power_rows(RowStep A)
     if (!iteration_start<sums_of<V>>(A, a, s)) return;
     double S[sums_of<V>] = {};
     while (sl < end) {
-        if (row != INF) emit_row<NORMLAP, V>(A, row, z, yr, wd, gb, a, s, S);
+        if (row != INF) emit_row<V>(A, row, z, yr, wd, gb, a, s, S);
         sl++;
         if (sl < end) slice();
     }
@@ -391,15 +390,15 @@ __global__ void k_pad_copy(uint32_t n, const double* __restrict__ x, V* __restri
     if (i <= n) y[i] = i < n ? (V)x[i] : (V)0;
 }
 
-template <bool NORMLAP, class V>
+template <class V>
 void launch(Ctx& c, const RowStep& A)
 {
     if (A.wfmt == W_UNIT)
-        k_power_rows<W_UNIT, NORMLAP, V><<<A.nblk, BLOCK, 0, c.stream>>>(A);
+        k_power_rows<W_UNIT, V><<<A.nblk, BLOCK, 0, c.stream>>>(A);
     else if (A.wfmt == W_U16)
-        k_power_rows<W_U16, NORMLAP, V><<<A.nblk, BLOCK, 0, c.stream>>>(A);
+        k_power_rows<W_U16, V><<<A.nblk, BLOCK, 0, c.stream>>>(A);
     else
-        k_power_rows<W_U32, NORMLAP, V><<<A.nblk, BLOCK, 0, c.stream>>>(A);
+        k_power_rows<W_U32, V><<<A.nblk, BLOCK, 0, c.stream>>>(A);
     MI_HIP(hipGetLastError());
 }
 
@@ -493,19 +492,12 @@ RowStep rows_step(Ctx& c, const DGraph& g, const RowPlan& p, const uint32_t* wde
     return A;
 }
 
-void launch_rows(Ctx& c, int normLap, bool f32, const RowStep& A)
+void launch_rows(Ctx& c, bool f32, const RowStep& A)
 {
-    if (f32) {
-        if (normLap)
-            launch<true, float>(c, A);
-        else
-            launch<false, float>(c, A);
-    } else {
-        if (normLap)
-            launch<true, double>(c, A);
-        else
-            launch<false, double>(c, A);
-    }
+    if (f32)
+        launch<float>(c, A);
+    else
+        launch<double>(c, A);
 }
 
 template <class V>

@@ -1,6 +1,7 @@
 // mi_small.hip -- the FP64 power iterations of consecutive small levels of a
 // hierarchy (eigensolve_kokkos.h:102-206, 1493-1558), coarsest first, in one
-// workgroup and one launch.
+// workgroup and one launch, under the plain Laplacian (the normalised one keeps
+// the order of sums of k_power_small_lds, mi_eigen.hip).
 //
 // A small level has up to a few thousand rows and takes hundreds of
 // iterations, each far shorter than a kernel launch.  What bounds one is the
@@ -230,7 +231,7 @@ __device__ __forceinline__ double inv_sqrt(double v)
 __host__ __device__ inline uint32_t span_of(uint32_t n) { return n < 64 ? 64u : n; }
 
 // The level's layout: order, slices, matrix, degrees.
-template <bool NORMLAP, int NWV>
+template <int NWV>
 __device__ __forceinline__ void build_layout(const SmallLevel& V, const SmallJob& J, double* pool, Layout& S)
 {
     using F = Form<NWV>;
@@ -409,7 +410,7 @@ __device__ __forceinline__ void build_layout(const SmallLevel& V, const SmallJob
         }
     }
     const uint32_t gb = max_all<NWV>(gbm, S.words + 64);  // (its barriers: every read of inv and the keys is done)
-    S.gb = NORMLAP ? 0u : (gb < 2u ? 2u : gb);
+    S.gb = gb < 2u ? 2u : gb;
     for (uint32_t i = tid; i < n; i += NT) S.wd[i] = J.deg[i];
     __syncthreads();
 }
@@ -479,15 +480,14 @@ __device__ __forceinline__ void share_sums(double (&sum)[3], double* red, bool o
 }
 
 // One row's y and its terms of the sums.
-template <bool NORMLAP>
 __device__ __forceinline__ double row_value(double z, double yr, uint32_t wd, uint32_t gb, double a, double s,
                                             double (&sum)[3], bool mine)
 {
     const double x = (yr - a) * s;
     const double ax = s * (z - a * (double)wd);
-    const double y = NORMLAP ? 0.5 * x + 0.5 * ax * (1.0 / (double)wd) : fma((double)(uint32_t)(gb - wd), x, ax);
+    const double y = fma((double)(uint32_t)(gb - wd), x, ax);
     const double ym = mine ? y : 0.0, xm = mine ? x : 0.0;
-    if (!NORMLAP) sum[0] += ym;
+    sum[0] += ym;
     sum[1] = fma(ym, ym, sum[1]);
     sum[2] = fma(xm, ym, sum[2]);
     return y;
@@ -497,7 +497,7 @@ __device__ __forceinline__ double row_value(double z, double yr, uint32_t wd, ui
 // slices follow one another at a fixed distance and their lengths fit two
 // scalar registers (one byte each); else the slice table is read along (a
 // fifth slower on meshes, but it keeps levels with long rows in registers).
-template <bool NORMLAP, int NWV, bool WIDE, bool UNI>
+template <int NWV, bool WIDE, bool UNI>
 __device__ __forceinline__ void iterate_regs(const SmallLevel& V, const Layout& S, const uint32_t* __restrict__ ent,
                                              double tol, Loop& Z)
 {
@@ -610,7 +610,7 @@ __device__ __forceinline__ void iterate_regs(const SmallLevel& V, const Layout& 
                     z0 = fma(w, yv[u], z0);
             }
             if (--left == 0) {
-                const double y = row_value<NORMLAP>(group_sum(z0 + z1, t), yr, wd, S.gb, a, s, sum, mine);
+                const double y = row_value(group_sum(z0 + z1, t), yr, wd, S.gb, a, s, sum, mine);
                 if (mine) yn[pos] = y;
                 z0 = z1 = 0.0;
                 if (UNI) pos += S.wstep * per;
@@ -655,7 +655,7 @@ __device__ __forceinline__ void load_group(const uint32_t* p, Words<WIDE>& q)
 }
 
 // Streamed form; `ent`: lane 0's first word of this wavefront's stream.
-template <bool NORMLAP, int NWV, bool WIDE>
+template <int NWV, bool WIDE>
 __device__ __forceinline__ void iterate_stream(const SmallLevel& V, const Layout& S, const uint32_t* __restrict__ ent,
                                                double tol, Loop& Z)
 {
@@ -687,7 +687,7 @@ __device__ __forceinline__ void iterate_stream(const SmallLevel& V, const Layout
             wd = S.wd[mine ? pos : 0u];
         };
         auto close = [&]() {
-            const double y = row_value<NORMLAP>(group_sum(z, t), yr, wd, S.gb, a, s, sum, mine);
+            const double y = row_value(group_sum(z, t), yr, wd, S.gb, a, s, sum, mine);
             if (mine) yn[pos] = y;
             z = 0.0;
             sl += S.wstep;
@@ -721,7 +721,7 @@ __device__ __forceinline__ void iterate_stream(const SmallLevel& V, const Layout
 // chain and leaves its place in the chain's state; the next one continues
 // with the same values.  A chain whose start another one computes (`after`)
 // waits for a launch that finds that one done.
-template <bool NORMLAP, int NWV>
+template <int NWV>
 __global__ void __launch_bounds__(NWV * WAVE, NWV / 4)
     k_small_chain(const SmallJob* __restrict__ jobs, uint32_t chunk, double tol)
 {
@@ -744,28 +744,20 @@ __global__ void __launch_bounds__(NWV * WAVE, NWV / 4)
         S.slice = slice;
         S.red = red;
         S.words = words;
-        build_layout<NORMLAP, NWV>(V, J, pool, S);
+        build_layout<NWV>(V, J, pool, S);
         if (st.iter == 0) {
-            // the start vector, orthogonalised against 1n = 1/sqrt(n) (normLap
-            // 0: u -= (u . 1n) 1n; 1: u -= (sum u D 1n / sum 1n D 1n) 1n) and
+            // the start vector, orthogonalised against 1n = 1/sqrt(n) and
             // normalised (eigensolve_kokkos.h:118-150)
             const double c = 1 / sqrt((double)n);
             const double* start = k == 0 ? J.start : J.v[(k - 1) & 1];
-            double p0 = 0.0, p1 = 0.0;
+            double p0 = 0.0;
             for (uint32_t i = tid; i < n; i += NT) {
                 const uint32_t r = J.ord[i];
                 const double u = start[V.vcmap ? V.vcmap[r] : r];
                 S.y[i] = u;
-                if (!NORMLAP) {
-                    p0 += u * c;
-                } else {
-                    const double d = (double)S.wd[i];
-                    p0 += u * d * c;
-                    p1 += c * d * c;
-                }
+                p0 += u * c;
             }
-            const double num = sum_all<NWV>(p0, red);
-            const double shift = NORMLAP ? num * c / sum_all<NWV>(p1, red) : num * c;
+            const double shift = sum_all<NWV>(p0, red) * c;
             double q = 0.0;
             for (uint32_t i = tid; i < n; i += NT) {
                 const double u = S.y[i] - shift;
@@ -800,20 +792,20 @@ __global__ void __launch_bounds__(NWV * WAVE, NWV / 4)
             if constexpr (F::STEPS > 0) {
                 if (S.regs) {
                     if (F::F64W && S.wide)
-                        iterate_regs<NORMLAP, NWV, F::F64W, false>(V, S, J.ent + 2 * WAVE * S.base, tol, Z);
+                        iterate_regs<NWV, F::F64W, false>(V, S, J.ent + 2 * WAVE * S.base, tol, Z);
                     else if (S.uni)
-                        iterate_regs<NORMLAP, NWV, false, true>(V, S, J.ent + WAVE * S.base, tol, Z);
+                        iterate_regs<NWV, false, true>(V, S, J.ent + WAVE * S.base, tol, Z);
                     else
-                        iterate_regs<NORMLAP, NWV, false, false>(V, S, J.ent + WAVE * S.base, tol, Z);
+                        iterate_regs<NWV, false, false>(V, S, J.ent + WAVE * S.base, tol, Z);
                 }
             }
             if (!S.regs) {
                 if (S.in_lds)
-                    iterate_stream<NORMLAP, NWV, false>(V, S, S.ent_l + WAVE * S.base, tol, Z);
+                    iterate_stream<NWV, false>(V, S, S.ent_l + WAVE * S.base, tol, Z);
                 else if (!S.wide)
-                    iterate_stream<NORMLAP, NWV, false>(V, S, J.ent + WAVE * S.base, tol, Z);
+                    iterate_stream<NWV, false>(V, S, J.ent + WAVE * S.base, tol, Z);
                 else
-                    iterate_stream<NORMLAP, NWV, true>(V, S, J.ent + 2 * WAVE * S.base, tol, Z);
+                    iterate_stream<NWV, true>(V, S, J.ent + 2 * WAVE * S.base, tol, Z);
             }
         }
         // the loop's outcome, for the wavefronts that took no part
@@ -877,23 +869,25 @@ uint64_t matrix_words(const DGraph& g)
 }
 
 template <int NWV>
-void launch_chain(Ctx& c, const SmallJob* jobs, unsigned grid, int normLap, double tol)
+void launch_chain(Ctx& c, const SmallJob* jobs, unsigned grid, double tol)
 {
-    if (normLap)
-        k_small_chain<true, NWV><<<grid, NWV * WAVE, 0, c.stream>>>(jobs, c.small_chunk, tol);
-    else
-        k_small_chain<false, NWV><<<grid, NWV * WAVE, 0, c.stream>>>(jobs, c.small_chunk, tol);
+    k_small_chain<NWV><<<grid, NWV * WAVE, 0, c.stream>>>(jobs, c.small_chunk, tol);
 }
 
 }  // namespace
 
-bool small_level(const Ctx& c, const DGraph& g, bool mixed)
+bool small_level(const Ctx& c, const DGraph& g, bool mixed, int normLap)
 {
+    if (normLap) return !mixed && small_lds_level(c, g);
     return !mixed && g.m > 0 && g.n <= SMALL_MAX_N && g.m <= std::min(c.small_max_m, SMALL_MAX_M);
 }
 
 void solve_small_chains(Ctx& c, std::vector<SmallChain>& chains, int normLap, double tol)
 {
+    if (normLap) {
+        solve_lds_chains(c, chains, normLap, tol);
+        return;
+    }
     // runs of levels of one workgroup size, each a job; a chain's runs follow
     // one another in launches of their own (`depth`)
     struct Run {
@@ -1008,11 +1002,11 @@ void solve_small_chains(Ctx& c, std::vector<SmallChain>& chains, int normLap, do
             const SmallJob* dj = reinterpret_cast<const SmallJob*>(dp) + i;
             const unsigned grid = (unsigned)(e - i);
             if (runs[i].waves == 4)
-                launch_chain<4>(c, dj, grid, normLap, tol);
+                launch_chain<4>(c, dj, grid, tol);
             else if (runs[i].waves == 8)
-                launch_chain<8>(c, dj, grid, normLap, tol);
+                launch_chain<8>(c, dj, grid, tol);
             else
-                launch_chain<16>(c, dj, grid, normLap, tol);
+                launch_chain<16>(c, dj, grid, tol);
             MI_HIP(hipGetLastError());
             i = e;
         }
