@@ -28,11 +28,13 @@
 //  - Register form (4 and 8 wavefronts): every wavefront's stream fits in
 //    registers and is read once per level; T the same for every row, or, when
 //    that makes a stream too long, growing with the row length.
-//  - Streamed form, for the others (long rows, many entries): T grows with the
-//    row length, the stream is read from LDS, or from global memory (L2) when
-//    it does not fit there, four steps at a time with the next four in flight.
-// Which one a level takes follows from its rows alone; the workgroup has 4, 8
-// or 16 wavefronts by the level's size (waves_of).  Every sum has a fixed
+//  - Streamed form (4 and 16 wavefronts), for the others (long rows, many
+//    entries): T grows with the row length, the stream is read from LDS, or
+//    from global memory (L2) when it does not fit there, four steps at a time
+//    with the next four in flight.
+// Which one a level takes follows from its rows and weights alone; the
+// workgroup has 4, 8 or 16 wavefronts by the level's size (waves_of), 16 also
+// where the registers of 8 turn out not to hold it.  Every sum has a fixed
 // order (the sort key ends in the row id), so results are bit-identical run
 // to run, and the same whether a level is solved alone, in a chain or in a
 // batch of chains.
@@ -57,7 +59,7 @@ constexpr uint32_t LEN_MAX = (1u << (32 - COL_BITS)) - 1u;
 constexpr uint32_t MAX_SLICES = 1152;
 constexpr uint32_t GROUP = 4;                 // steps per load group
 
-// The two workgroup sizes.
+// The workgroup sizes.
 template <int NWV>
 struct Form;
 template <>
@@ -118,6 +120,7 @@ struct SmallResult {
     unsigned long long iters;
     unsigned long long ticks;
     uint32_t max_reached, done;
+    uint32_t to16, pad;  // to16: the registers of eight wavefronts do not hold the level
 };
 
 // Where a launch that ran out of its iterations left the loop.
@@ -130,7 +133,7 @@ struct SmallState {
 struct SmallJob {
     const SmallLevel* lv;
     SmallResult* res;
-    uint32_t nlv;
+    uint32_t nlv, waves;
     const double* start;
     const SmallResult* after;  // the last level of the chain that computes `start` (null: none)
     double* v[2];   // the vector of level k of the chain goes to v[k & 1]
@@ -721,6 +724,12 @@ __device__ __forceinline__ void iterate_stream(const SmallLevel& V, const Layout
 // chain and leaves its place in the chain's state; the next one continues
 // with the same values.  A chain whose start another one computes (`after`)
 // waits for a launch that finds that one done.
+// A level that the registers of eight wavefronts do not hold (rows of hundreds
+// of entries whose padding does not fit, or weights past 16 bits) is left to
+// sixteen, launched in the next round: eight hide its loads worse when they
+// stream it (R-MAT level of 388 vertices and 49,268 entries 15.6 us per
+// iteration against 10.0; 400 and 37,654 with heavy weights 11.4 against 7.6;
+// 200 and 15,374 4.6 against 3.4).
 template <int NWV>
 __global__ void __launch_bounds__(NWV * WAVE, NWV / 4)
     k_small_chain(const SmallJob* __restrict__ jobs, uint32_t chunk, double tol)
@@ -736,7 +745,11 @@ __global__ void __launch_bounds__(NWV * WAVE, NWV / 4)
     const uint32_t tid = threadIdx.x, wid = uniform(tid / WAVE);
     SmallState st = *J.st;
     uint32_t budget = chunk;
-    for (uint32_t k = st.level; k < J.nlv; k++) {
+    uint32_t k = st.level;
+    for (; k < J.nlv; k++) {
+        // (sixteen wavefronts launched for a run of eight: the levels passed on)
+        if (NWV == 8 && J.res[k].to16) break;
+        if (NWV == 16 && J.waves == 8 && !J.res[k].to16) break;
         const SmallLevel V = J.lv[k];
         const uint32_t n = V.n;
         const unsigned long long tick = wall_clock64();
@@ -745,6 +758,10 @@ __global__ void __launch_bounds__(NWV * WAVE, NWV / 4)
         S.red = red;
         S.words = words;
         build_layout<NWV>(V, J, pool, S);
+        if (NWV == 8 && !S.regs) {
+            if (tid == 0) J.res[k].to16 = 1u;
+            break;
+        }
         if (st.iter == 0) {
             // the start vector, orthogonalised against 1n = 1/sqrt(n) and
             // normalised (eigensolve_kokkos.h:118-150)
@@ -799,13 +816,15 @@ __global__ void __launch_bounds__(NWV * WAVE, NWV / 4)
                         iterate_regs<NWV, false, false>(V, S, J.ent + WAVE * S.base, tol, Z);
                 }
             }
-            if (!S.regs) {
-                if (S.in_lds)
-                    iterate_stream<NWV, false>(V, S, S.ent_l + WAVE * S.base, tol, Z);
-                else if (!S.wide)
-                    iterate_stream<NWV, false>(V, S, J.ent + WAVE * S.base, tol, Z);
-                else
-                    iterate_stream<NWV, true>(V, S, J.ent + 2 * WAVE * S.base, tol, Z);
+            if constexpr (NWV != 8) {
+                if (!S.regs) {
+                    if (S.in_lds)
+                        iterate_stream<NWV, false>(V, S, S.ent_l + WAVE * S.base, tol, Z);
+                    else if (!S.wide)
+                        iterate_stream<NWV, false>(V, S, J.ent + WAVE * S.base, tol, Z);
+                    else
+                        iterate_stream<NWV, true>(V, S, J.ent + 2 * WAVE * S.base, tol, Z);
+                }
             }
         }
         // the loop's outcome, for the wavefronts that took no part
@@ -856,7 +875,10 @@ __global__ void __launch_bounds__(NWV * WAVE, NWV / 4)
         st.iter = 0;
         __syncthreads();
     }
-    if (tid == 0) J.st->level = J.nlv;
+    if (tid == 0) {
+        J.st->level = k;
+        J.st->iter = st.iter;
+    }
 }
 
 // Matrix words of a level outside LDS at most: every class of rows pads its
@@ -964,6 +986,7 @@ void solve_small_chains(Ctx& c, std::vector<SmallChain>& chains, int normLap, do
         q.lv = reinterpret_cast<const SmallLevel*>(dp + o_lv) + first[r.chain] + r.k0;
         q.res = dres + first[r.chain] + r.k0;
         q.nlv = L;
+        q.waves = (uint32_t)r.waves;
         q.start = r.k0 ? last[r.chain] : ch.start;
         q.after = r.k0 ? q.res - 1 : nullptr;
         double* out = r.k1 == ch.lv.size() ? ch.out : w + r.nmax;
@@ -993,6 +1016,7 @@ void solve_small_chains(Ctx& c, std::vector<SmallChain>& chains, int normLap, do
     }
     MI_HIP(hipMemcpyAsync(table.get(), host.data(), bytes, hipMemcpyHostToDevice, c.stream));
     const size_t res_bytes = nlv * sizeof(SmallResult);
+    bool passed_on = false;  // some level awaits sixteen wavefronts
     for (unsigned long long launched = 0;; launched += c.small_chunk) {
         MI_CHECK(launched / depths <= cap + c.small_chunk, ST_INTERNAL,
                  "power iteration did not stop at its iteration cap");
@@ -1005,15 +1029,19 @@ void solve_small_chains(Ctx& c, std::vector<SmallChain>& chains, int normLap, do
                 launch_chain<4>(c, dj, grid, tol);
             else if (runs[i].waves == 8)
                 launch_chain<8>(c, dj, grid, tol);
-            else
-                launch_chain<16>(c, dj, grid, tol);
+            // (before any level is passed on: none of that size)
+            if (runs[i].waves == 16 || (runs[i].waves == 8 && passed_on)) launch_chain<16>(c, dj, grid, tol);
             MI_HIP(hipGetLastError());
             i = e;
         }
         MI_HIP(hipMemcpyAsync(hres, dres, res_bytes, hipMemcpyDeviceToHost, c.stream));
         MI_HIP(hipStreamSynchronize(c.stream));
         bool all = true;
-        for (size_t k = 0; k < nlv && all; k++) all = hres[k].done != 0;
+        passed_on = false;
+        for (size_t k = 0; k < nlv; k++) {
+            all = all && hres[k].done;
+            passed_on = passed_on || (hres[k].to16 && !hres[k].done);
+        }
         if (all) break;
     }
     int khz = 0;

@@ -110,6 +110,58 @@ def test_small_level_against_numpy(ctx, name, normLap):
         assert it == 1 or abs(dots[-2] - dots[-3]) > TOL * (1 - 1e-6)
 
 
+def _blocks(sizes, rng, wmax):
+    """Complete graphs joined in a path by one edge each: dense, and slow to
+    converge."""
+    us, vs, at = [], [], 0
+    for k in sizes:
+        i, j = np.triu_indices(k, 1)
+        us += [i + at, [at]]
+        vs += [j + at, [at + k]]
+        at += k
+    u, v = np.concatenate(us[:-1]), np.concatenate(vs[:-1])
+    w = rng.integers(1, 9, len(u))
+    w[::97] = wmax
+    return graphs.from_edges(at, u, v, w, lcc=False)
+
+
+@pytest.mark.parametrize("sizes,wmax", [
+    ([102] * 5, 9),           # 128 steps per wavefront: eight hold the level in registers
+    ([104] * 5, 9),           # 144: sixteen
+    ([90, 80, 70], 65535),    # the largest weight of the register form
+    ([90, 80, 70], 65536)])   # ... past it
+def test_level_passed_on_to_sixteen_wavefronts(ctx, sizes, wmax):
+    """Levels whose rows or weights the registers of eight wavefronts do not
+    hold go on in sixteen, alone and as the last of a chain: against numpy, and
+    launches of one, three and 8192 iterations give the same bits."""
+    rng = np.random.default_rng(11)
+    rp, col, w = _blocks(sizes, rng, wmax)
+    n = len(rp) - 1
+    u0 = rng.uniform(-1, 1, n)
+    g = ctx.graph(rp, col, w)
+    runs, sols = [], []
+    try:
+        for chunk in (0, 3, 1):
+            ctx.set_small_levels(1 << 17, chunk)
+            u, it, most = g.power_iter(u0, tol=TOL)
+            assert not most
+            runs.append((u, it))
+            H = g.hierarchy(5)
+            ev, st, _ = H.fiedler(9, tol=TOL)
+            sols.append((ev, st["level_iters"]))
+            H.close()
+    finally:
+        ctx.set_small_levels()
+        g.close()
+    for u, it in runs[1:]:
+        assert it == runs[0][1] and np.array_equal(u, runs[0][0])
+    for ev, iters in sols[1:]:
+        assert iters == sols[0][1] and np.array_equal(ev, sols[0][0])
+    hu, dots = _host(rp, col, w, u0, 0, runs[0][1])
+    assert np.linalg.norm(runs[0][0] - hu) <= 1e-11
+    assert abs(dots[-1] - dots[-2]) <= TOL * (1 + 1e-6)
+
+
 def test_rows_without_entries(ctx):
     """Isolated vertices (their rows come last in the layout, in slices of no
     steps): y = (gb - 0) x there."""
