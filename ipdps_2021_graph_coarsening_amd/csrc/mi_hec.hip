@@ -1168,9 +1168,36 @@ __global__ void k_match_compact(uint32_t len, const uint32_t* __restrict__ list,
 // wait of the host per step, about 110 us however short the list (the maps of
 // all 15 levels of a random geometric graph of 150,001 vertices: 6.2 ms by
 // launches, 3.5 ms so).  LANES lanes share the row of a slot when it looks for
-// its next neighbour.
+// its next neighbour, a whole wavefront a row of more than LONG entries.
 constexpr uint32_t MATCH_ONE_WG = 4096;
+// The rows of the list are read in every round, by one CU instead of all: lists
+// whose rows hold more entries stay with the launches until they have shrunk
+// (hierarchies of random graphs of 4000 vertices, ms, by launches, with this
+// line at 2^16, 2^18, 2^20 entries and without one: 0.63 M entries 6.27, 4.24,
+// 4.25, 4.65, 4.63; 1.5 M 7.7, 5.7, 5.5, 8.0, 8.5; 5.3 M 14.7, 12.7, 12.4, 21.8,
+// 84.4; R-MAT of 2^12, 96,000 entries 10.1, 4.8, 4.7, 4.7, 4.7; hubs of 10,000 to
+// 100,000 entries on sparse graphs 6.3 to 12, 4.2 to 8.7 wherever it lies).
+constexpr uint32_t MATCH_ONE_WG_M = 1u << 18;
 constexpr int MATCH_BLOCK = 1024;
+
+// cnt[1] = entries of the rows of a list of cnt[0] slots (more than MATCH_ONE_WG: INF)
+__global__ void __launch_bounds__(MATCH_BLOCK) k_match_entries(const uint32_t* __restrict__ list,
+                                                               const uint32_t* __restrict__ rowptr, uint32_t* cnt)
+{
+    __shared__ uint32_t lds[MATCH_BLOCK / WAVE];
+    const uint32_t len = cnt[0], lane = threadIdx.x & (WAVE - 1);
+    uint32_t sum = 0;
+    if (len <= MATCH_ONE_WG)
+        for (uint32_t k = threadIdx.x; k < len; k += MATCH_BLOCK) sum += rowptr[list[k] + 1] - rowptr[list[k]];
+    sum = wave_sum_u32(sum);
+    if (lane == 0) lds[threadIdx.x / WAVE] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        sum = 0;
+        for (int j = 0; j < MATCH_BLOCK / WAVE; j++) sum += lds[j];
+        cnt[1] = len <= MATCH_ONE_WG ? sum : INF;
+    }
+}
 
 struct MatchTail {
     uint32_t len, nc, cap;  // cap: rounds at most
@@ -1189,9 +1216,9 @@ struct MatchTail {
     uint32_t* out;  // ids given, swap, 0 or what went wrong (1: only self-loops left, 2: did not end)
 };
 
-template <int LANES>
 __global__ void __launch_bounds__(MATCH_BLOCK) k_match_tail(MatchTail a)
 {
+    constexpr uint32_t LANES = 8, LONG = 64;
     __shared__ uint32_t wsum[2][MATCH_BLOCK / WAVE], undecided;
     const uint32_t t = threadIdx.x, lane = t & (WAVE - 1), wv = t / WAVE;
     uint32_t len = a.len, nc = a.nc, err = 0;
@@ -1282,29 +1309,45 @@ __global__ void __launch_bounds__(MATCH_BLOCK) k_match_tail(MatchTail a)
         }
         nc += pairs;
         __syncthreads();
-        for (uint32_t k = t / LANES; k < len; k += MATCH_BLOCK / LANES) {
-            const uint32_t u = la[k], l = t % LANES;
-            const bool open = a.vcmap[u] == INF;
-            uint64_t key = 0;
-            bool any = false;
-            if (open) {
-                for (uint32_t e = a.rowptr[u] + l, r1 = a.rowptr[u + 1]; e < r1; e += LANES) {
+        // (whole wavefronts: idle lanes past the last slot take part in the exchanges)
+        for (uint32_t k0 = 0; k0 < len; k0 += MATCH_BLOCK / LANES) {
+            const uint32_t k = k0 + t / LANES, l = t % LANES;
+            const uint32_t u = k < len ? la[k] : 0u;
+            const bool open = k < len && a.vcmap[u] == INF;
+            const uint32_t r0 = open ? a.rowptr[u] : 0u, r1 = open ? a.rowptr[u + 1] : 0u;
+            const bool is_long = r1 - r0 > LONG;
+            // the largest (key, entry), + 1, of this lane's entries; 0: none
+            // (e < 2^32 - 1 keeps it from wrapping)
+            const auto scan = [&](uint32_t e, uint32_t end, uint32_t step) {
+                uint64_t best = 0;
+                for (; e < end; e += step) {
                     const uint32_t v = a.col[e];
                     if (a.vcmap[v] != INF) continue;
                     const uint32_t kv = a.level == 1 ? a.pos[v] : (a.w ? a.w[e] : 1u);
-                    const uint64_t x = ((uint64_t)kv << 32) | e;
-                    key = (!any || x > key) ? x : key;
-                    any = true;
+                    const uint64_t x = (((uint64_t)kv << 32) | e) + 1;
+                    best = x > best ? x : best;
                 }
-            }
-            // (key + 1 below: 0 says none; e < 2^32 - 1 keeps it from wrapping)
-            uint64_t best = any ? key + 1 : 0;
+                return best;
+            };
+            uint64_t best = is_long ? 0 : scan(r0 + l, r1, LANES);
 #pragma unroll
             for (int o = LANES / 2; o > 0; o >>= 1) {
                 const uint64_t x = __shfl_xor(best, o, WAVE);
                 best = x > best ? x : best;
             }
-            if (l == 0) {
+            for (unsigned long long todo = __ballot(is_long && l == 0); todo; todo &= todo - 1) {
+                const int src = __builtin_ctzll(todo);
+                const uint32_t s0 = (uint32_t)__builtin_amdgcn_readlane((int)r0, src);
+                const uint32_t s1 = (uint32_t)__builtin_amdgcn_readlane((int)r1, src);
+                uint64_t b = scan(s0 + lane, s1, WAVE);
+#pragma unroll
+                for (int o = WAVE / 2; o > 0; o >>= 1) {
+                    const uint64_t x = __shfl_xor(b, o, WAVE);
+                    b = x > b ? x : b;
+                }
+                if ((int)lane == src) best = b;
+            }
+            if (k < len && l == 0) {
                 a.keep[k] = best ? 1u : 0u;
                 if (best) a.hn[u] = a.col[(uint32_t)(best - 1)];
             }
@@ -2284,17 +2327,14 @@ static uint32_t match_rounds(Ctx& c, const DGraph& g, int level, const uint32_t*
     fill_u32(c, vcmap, n, INF);
     uint32_t len = n, nc = 0;
     int swap = 1, idle = 0;
+    uint32_t entries = g.m;  // of the listed rows, or more
     for (uint32_t round = 0; len > 0; round++) {
         MI_CHECK(round <= 2ull * n + 4, ST_INTERNAL, "matching rounds did not end");
-        if (len <= MATCH_ONE_WG) {
+        if (len <= MATCH_ONE_WG && entries <= MATCH_ONE_WG_M) {
             const MatchTail a{len,     nc,      (uint32_t)(2ull * n + 4 - round), swap, idle, level,
                               g.R(),   g.Cc(),  g.W(),         pos,           la.get(),      lb.get(),
                               hn,      vcmap,   B.est.get(),   B.first.get(), B.flag.get(),  B.cnt.get()};
-            // (a lane or a few per short row; long rows by whole wavefronts)
-            if (g.m >= 32ull * n)
-                k_match_tail<WAVE><<<1, MATCH_BLOCK, 0, c.stream>>>(a);
-            else
-                k_match_tail<8><<<1, MATCH_BLOCK, 0, c.stream>>>(a);
+            k_match_tail<<<1, MATCH_BLOCK, 0, c.stream>>>(a);
             MI_HIP(hipGetLastError());
             uint32_t h[3] = {0, 0, 0};
             read_words(c, B.cnt.get(), h, 12);
@@ -2313,14 +2353,21 @@ static uint32_t match_rounds(Ctx& c, const DGraph& g, int level, const uint32_t*
         scan_exclusive_u32(c, B.flag.get(), B.rank.get(), len, B.cnt.get() + 2);
         k_match_compact<<<grid1(len), BLOCK, 0, c.stream>>>(len, la.get(), B.flag.get(), B.rank.get(), lb.get());
         MI_HIP(hipGetLastError());
-        uint32_t nl = 0;
-        read_words(c, B.cnt.get() + 2, &nl, 4);
+        uint32_t nl[2] = {0, 0};
+        if (g.m > MATCH_ONE_WG_M) {
+            k_match_entries<<<1, MATCH_BLOCK, 0, c.stream>>>(lb.get(), g.R(), B.cnt.get() + 2);
+            MI_HIP(hipGetLastError());
+            read_words(c, B.cnt.get() + 2, nl, 8);
+            entries = nl[1];
+        } else {
+            read_words(c, B.cnt.get() + 2, nl, 4);
+        }
         idle = pairs ? 0 : idle + 1;
         // three rounds in a row without a pair: the last two held the same
         // edges under both orderings, so only self-loops are left (the
         // reference loops for ever)
-        MI_CHECK(!(idle >= 3 && nl > 0), ST_ARG, "matching: only self-loops left");
-        len = nl;
+        MI_CHECK(!(idle >= 3 && nl[0] > 0), ST_ARG, "matching: only self-loops left");
+        len = nl[0];
         swap ^= 1;
         la.swap(lb);
     }

@@ -126,6 +126,40 @@ def test_dropin_match(tmp_path, fm):
         assert [l["number-vertices"] for l in t["coarse-levels"]] == [int(x) for x in o["levels_n"]][::-1]
 
 
+def _hubs(n, degrees, rng):
+    """A path plus rows of the given numbers of entries."""
+    us, vs = [np.arange(n - 1)], [np.arange(1, n)]
+    for i, d in enumerate(degrees):
+        h = 3 + i * (n // len(degrees))
+        to = rng.choice(np.delete(np.arange(n), [h - 1, h, h + 1]), d - 2, replace=False)
+        us.append(np.full(d - 2, h))
+        vs.append(to)
+    u, v = np.concatenate(us), np.concatenate(vs)
+    return graphs.from_edges(n, u, v, rng.integers(1, 4, len(u)), lcc=False)
+
+
+@pytest.mark.parametrize("n,degrees", [
+    (512, None), (513, None),   # complete: 261,632 and 262,656 entries, on both sides of 2^18
+    (4000, (63, 64, 65, 66, 3000)), (4100, (64, 65, 4000))])  # rows by eight lanes and by a wavefront
+def test_match_long_rows_and_dense_levels(mt, n, degrees):
+    """Lists whose rows hold more than 2^18 entries stay with the launches
+    until they have shrunk; rows of more than 64 entries are read by a whole
+    wavefront."""
+    rng = np.random.default_rng(n)
+    if degrees is None:
+        u, v = np.triu_indices(n, 1)
+        rp, col, w = graphs.from_edges(n, u, v, rng.integers(1, 9, len(u)), lcc=False)
+        assert (len(col) > 1 << 18) == (n == 513)
+    else:
+        rp, col, w = _hubs(n, degrees, rng)
+    g = mt.graph(rp, col, w)
+    for level in (1, 2):
+        vc, nc, _, _ = g.hec_level(level, 7)
+        ovc, onc, _ = oracle.coarsen_match(level, rp, col, w, 7)
+        assert nc == onc and np.array_equal(vc, ovc)
+    g.close()
+
+
 @pytest.mark.parametrize("n", [2, 63, 1024, 1025, 4095, 4096, 4097, 6000])
 def test_match_list_ends_in_one_workgroup(mt, n):
     """Lists of at most 4096 slots run their rounds in one workgroup (1024
