@@ -92,8 +92,10 @@ __global__ void k_scatter_pos(const uint32_t* __restrict__ vperm, uint32_t n, ui
 // hierarchy draws from the same seed, so a coarser level's keys are the first
 // of the finer level's and its argsort is that one without the vertices from n
 // on.  Workgroup b takes PERM_CH entries; k_perm_filter sums the counts of the
-// workgroups before it (at most a few thousand) itself.
+// workgroups before it itself, or, where there are more than PERM_SUMS of them
+// (2 million vertices; that reading grows with their square), gets the sums.
 constexpr uint32_t PERM_CH = 8 * BLOCK;
+constexpr uint32_t PERM_SUMS = 1024;
 __global__ void __launch_bounds__(BLOCK) k_perm_count(uint32_t np, const uint32_t* __restrict__ prev, uint32_t n,
                                                       uint32_t* __restrict__ counts)
 {
@@ -110,13 +112,17 @@ __global__ void __launch_bounds__(BLOCK) k_perm_count(uint32_t np, const uint32_
 }
 
 __global__ void __launch_bounds__(BLOCK) k_perm_filter(uint32_t np, const uint32_t* __restrict__ prev, uint32_t n,
-                                                       const uint32_t* __restrict__ counts,
+                                                       const uint32_t* __restrict__ counts, bool sums,
                                                        uint32_t* __restrict__ vperm, uint32_t* __restrict__ pos)
 {
     __shared__ uint32_t lds[BLOCK / WAVE], base, wcnt[BLOCK / WAVE];
     uint32_t before = 0;
-    for (uint32_t b = threadIdx.x; b < blockIdx.x; b += BLOCK) before += counts[b];
-    before = block_sum_u32(before, lds);
+    if (sums) {
+        before = counts[blockIdx.x];
+    } else {
+        for (uint32_t b = threadIdx.x; b < blockIdx.x; b += BLOCK) before += counts[b];
+        before = block_sum_u32(before, lds);
+    }
     if (threadIdx.x == 0) base = before;
     // a wavefront takes consecutive entries, 64 at a time
     constexpr uint32_t STEPS = PERM_CH / BLOCK;
@@ -2721,7 +2727,11 @@ uint32_t hec_map(Ctx& c, const DGraph& g, const uint32_t* roc, int level, uint64
         DBuf<uint32_t> counts(&c.pool, nb);
         k_perm_count<<<nb, BLOCK, 0, c.stream>>>(hs.n, hs.vperm.get(), n, counts.get());
         MI_HIP(hipGetLastError());
-        k_perm_filter<<<nb, BLOCK, 0, c.stream>>>(hs.n, hs.vperm.get(), n, counts.get(), next.get(), pos.get());
+        const bool sums = nb > PERM_SUMS;
+        DBuf<uint32_t> at(&c.pool, sums ? nb : 1);
+        if (sums) scan_exclusive_u32(c, counts.get(), at.get(), nb, nullptr);
+        k_perm_filter<<<nb, BLOCK, 0, c.stream>>>(hs.n, hs.vperm.get(), n, sums ? at.get() : counts.get(), sums,
+                                                  next.get(), pos.get());
         MI_HIP(hipGetLastError());
         hs.vperm = std::move(next);
     } else {

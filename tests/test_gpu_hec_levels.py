@@ -3,6 +3,8 @@ hierarchy draws the random stream once and filters each level's permutation
 out of the finer level's (csrc/mi_hec.hip, 2048 entries per workgroup), a
 single level draws and sorts its own.  Integers, compared exactly; each
 hierarchy's own levels against the oracle: test_gpu_parity.py."""
+import itertools
+
 import numpy as np
 import pytest
 
@@ -12,12 +14,14 @@ from ipdps_2021_graph_coarsening_amd import graphs
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("variant", [0, 1, 3, 4])
-@pytest.mark.parametrize("n", [51, 255, 2047, 2048, 2049, 4097, 70001])
+@pytest.mark.parametrize("n,variant", [
+    *itertools.product([51, 255, 2047, 2048, 2049, 4097, 70001], [0, 1, 3, 4]),
+    (2048 * 1024, 0), (2048 * 1024 + 1, 0)])  # 1024 workgroups, and one more (their counts are scanned)
 def test_levels_one_by_one(ctx, n, variant):
     rng = np.random.default_rng(n)
     k = np.arange(n - 1)
-    u, v = np.concatenate([k, rng.integers(0, n, n)]), np.concatenate([k + 1, rng.integers(0, n, n)])
+    extra = n if n < 1 << 20 else n // 50
+    u, v = np.concatenate([k, rng.integers(0, n, extra)]), np.concatenate([k + 1, rng.integers(0, n, extra)])
     rp, col, w = graphs.from_edges(n, u, v, rng.integers(1, 9, len(u)), lcc=False)
     ctx.set_coarsening(variant)
     try:
