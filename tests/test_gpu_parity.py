@@ -405,6 +405,31 @@ def test_eigenvalue_log_vs_oracle(ctx, weighted):
     assert st1["eigen_log"] is None
 
 
+@pytest.mark.parametrize("weighted", [False, True])
+def test_eigenvalue_log_of_a_small_finest_level(ctx, weighted):
+    """A level without a plan has its product taken from the CSR rows: rows by
+    16 lanes, of more than 512 entries by a workgroup (511, 512, 513 and 4000
+    here, two of them in one workgroup).  Tolerances as above."""
+    rng = np.random.default_rng(2)
+    n = 4203
+    us, vs = [np.arange(n - 1)], [np.arange(1, n)]
+    for h, d in ((10, 511), (14, 512), (18, 513), (22, 4000), (4202, 600)):
+        to = rng.choice(np.arange(100, 4150), d - (2 if h < n - 1 else 1), replace=False)
+        us.append(np.full(len(to), h))
+        vs.append(to)
+    u, v = np.concatenate(us), np.concatenate(vs)
+    rp, col, w = graphs.from_edges(n, u, v, rng.integers(1, 9, len(u)) if weighted else None, lcc=False)
+    assert sorted(np.diff(rp))[-5:] == [511, 512, 513, 600, 4000]
+    g = ctx.graph(rp, col, w)
+    ev, st, _ = g.hierarchy(2).fiedler(55)
+    el = st["eigen_log"]
+    oe, omn, omx = oracle.eigenvalue_log(rp, col, w, ev)
+    assert abs(el["eigenvalue"] - oe) <= 1e-9 * abs(oe)
+    assert abs(el["min"] - omn) <= 1e-9 * max(1.0, abs(omn))
+    assert abs(el["max"] - omx) <= 1e-9 * max(1.0, abs(omx))
+    g.close()
+
+
 @pytest.mark.parametrize("name", ["path40", "path3000", "star", "disconnected", "rgg"])
 def test_partition_graph_edge_cases(ctx, name):
     rng = np.random.default_rng(1)
