@@ -113,8 +113,9 @@ int mi_ctx_set_precision(mi_ctx* ctx, int mixed, uint32_t min_entries);
    iteration in one workgroup, consecutive such levels in one launch, chunk
    iterations per launch at most (0: 8192),
    instead of launches per iteration.  Same stop rule and
-   result bookkeeping; the sums are added in another order.  Under the
-   normalised Laplacian: levels of at most 16384 vertices and max_entries
+   result bookkeeping; the sums are added in another order.  So do levels of
+   up to 8192 vertices and 36864 entries with a row of more than 128, a launch
+   each.  Under the normalised Laplacian: levels of at most 16384 vertices and max_entries
    entries, a launch each.  No counterpart in the reference. */
 int mi_ctx_set_small_levels(mi_ctx* ctx, uint32_t max_entries, uint32_t chunk);
 /* enable != 0 (the default): a level above the finest with at least

@@ -1477,6 +1477,7 @@ __global__ void __launch_bounds__(LBLOCK) k_power_small(StepArgs A, double* buf0
 // sum 1n D 1n) 1n) and normalised, with the sums taken in this workgroup.
 constexpr uint32_t SMALL_LDS = 18432;  // doubles (144 KiB)
 constexpr uint32_t SMALL_RPT = 8;      // rows per thread at most (instances for 4 and 8)
+constexpr uint32_t LDS_LEVEL_M = 36864;  // entries of a plain level at most (see power_iter)
 
 // Sum of v over the workgroup, in every thread (a fixed order); red[0] is
 // reused, behind barriers on both sides.
@@ -2838,18 +2839,21 @@ void power_iter(Ctx& c, const DGraph& g, double* d_u, int normLap, double tol, P
     const uint32_t n = g.n;
     MI_CHECK(n > 0, ST_ARG, "empty level");
     auto t0 = std::chrono::steady_clock::now();
-    if (small_level(c, g, mixed, normLap)) {
+    const auto one_workgroup = [&](auto&& solve) {
         std::vector<SmallChain> one(1);
         one[0].lv.resize(1);
         one[0].lv[0].g = &g;
         one[0].start = one[0].out = d_u;
-        solve_small_chains(c, one, normLap, tol);
+        solve(c, one, normLap, tol);
         if (eig_log && !normLap) eigen_log_level(c, g, d_u, eig_log);
         if (st) {
             st->iters = one[0].lv[0].iters;
             st->max_reached = one[0].lv[0].max_reached;
             st->ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
         }
+    };
+    if (small_level(c, g, mixed, normLap)) {
+        one_workgroup(solve_small_chains);
         return;
     }
     DBuf<uint32_t> wdeg(&c.pool, n), gb(&c.pool, 1);
@@ -2857,6 +2861,16 @@ void power_iter(Ctx& c, const DGraph& g, double* d_u, int normLap, double tol, P
     DBuf<float> f0, f1;   // ... in the mixed form
     LevelPlan plan;
     plan_level(c, g, plan, mixed, normLap);
+    // Past the rows that mi_small.hip takes and with a row that mi_rows.hip does
+    // not: few entries are streamed faster by one workgroup than by two launches
+    // (us per iteration, one workgroup and two launches: 7,700 vertices and
+    // 20,000 entries 10.1 and 14.4, 28,000 11.9 and 14.4, 36,500 13.9 and 14.1,
+    // 39,600 15.6 and 13.9; 7,400 and 62,000 20 and 15).
+    if (!normLap && !mixed && !plan.rows.on && g.m <= LDS_LEVEL_M && small_lds_level(c, g)) {
+        plan = LevelPlan();
+        one_workgroup(solve_lds_chains);
+        return;
+    }
     weighted_degree(c, g, plan, wdeg.get(), gb.get());
 
     // vec1 = 1, normalised: every entry is 1/sqrt(n) (n is exact in FP64)

@@ -576,7 +576,7 @@ def test_context_destroyed_before_its_objects():
 
 
 @pytest.mark.parametrize("normLap", [0, 1])
-@pytest.mark.parametrize("case", ["er3000w", "grid64", "rmat11w_hubs", "grid80", "grid100"])
+@pytest.mark.parametrize("case", ["er3000w", "grid64", "rmat11w_hubs", "grid80", "grid100", "hub8192", "hub8000"])
 def test_small_level_workgroup_vs_steps_and_oracle(ctx, case, normLap):
     """The one-workgroup loop of small levels (vectors in LDS up to 8192
     vertices, 4 or 8 rows per thread: grid80 takes the 8-row form, grid100
@@ -594,6 +594,14 @@ def test_small_level_workgroup_vs_steps_and_oracle(ctx, case, normLap):
         rp, col, w = graphs.grid2d(80)
     elif case == "grid100":
         rp, col, w = graphs.grid2d(100)
+    elif case.startswith("hub"):  # the most entries that a plain level past 7168 vertices has in that form, and more
+        n, m = int(case[3:]), 36864 if case == "hub8192" else 36866
+        us, vs = [np.arange(n - 1), np.zeros(129, np.int64)], [np.arange(1, n), np.arange(2, 131)]
+        k = np.arange(m // 2 - n + 1 - 129)
+        us.append(200 + k % (n - 400))
+        vs.append(us[-1] + 2 + k // (n - 400))
+        rp, col, w = graphs.from_edges(n, np.concatenate(us), np.concatenate(vs), rng.integers(1, 9, m // 2), lcc=False)
+        assert len(col) == m
     else:
         rp, col, w = graphs.rmat(11, 16, seed=4)
     u0 = rng.random(len(rp) - 1)
