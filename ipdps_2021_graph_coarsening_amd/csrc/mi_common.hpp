@@ -243,14 +243,23 @@ __device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v)
     return v;
 }
 
+// largest of the 64 lanes' values, in every lane (all lanes active)
 __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v)
 {
-#pragma unroll
-    for (int o = WAVE / 2; o > 0; o >>= 1) {
-        uint32_t t = __shfl_xor(v, o, WAVE);
-        v = t > v ? t : v;
+    // (a lane without a source keeps its own value)
+#define MI_STEP(CTRL, ROWS)                                                                             \
+    {                                                                                                   \
+        const uint32_t t = (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, ROWS, 0xf, false); \
+        v = t > v ? t : v;                                                                              \
     }
-    return v;
+    MI_STEP(0x111, 0xf)  // row_shr:1, 2, 4, 8: lane 15 of each row of 16 holds the row's
+    MI_STEP(0x112, 0xf)
+    MI_STEP(0x114, 0xf)
+    MI_STEP(0x118, 0xf)
+    MI_STEP(0x142, 0xa)  // row_bcast:15, :31: lane 63 holds all
+    MI_STEP(0x143, 0xc)
+#undef MI_STEP
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, WAVE - 1);
 }
 
 // Max over a block of BLOCK threads; result valid in every thread.

@@ -462,7 +462,7 @@ struct StepArgs {
     double c;
     double tol;
     unsigned long long iter_max;
-    int mode;  // 0: loop iteration, 1: one shifted product (a = 0, s = 1), 2: plain A x
+    int mode;  // 0: loop iteration, 1: one shifted product (a = 0, s = 1)
     uint32_t* cnt;
     double* scal;
     unsigned long long* niter;
@@ -1113,11 +1113,10 @@ __global__ void __launch_bounds__(LBLOCK) k_power_stream_lds(StepArgs A)
     }
 }
 
-// y_r from the row sum (the shifted product of the reference, or A x in mode 2)
+// y_r from the row sum (the shifted product of the reference)
 template <bool NORMLAP>
-__device__ __forceinline__ double shifted(const StepArgs& A, double spmv, double xr, uint32_t wd, uint32_t gb)
+__device__ __forceinline__ double shifted(double spmv, double xr, uint32_t wd, uint32_t gb)
 {
-    if (A.mode == 2) return spmv;
     if (!NORMLAP) return (double)(uint32_t)(gb - wd) * xr + spmv;
     return 0.5 * xr + 0.5 * spmv * (1.0 / (double)wd);
 }
@@ -1236,7 +1235,7 @@ __global__ void __launch_bounds__(BLOCK) k_power_finish(StepArgs A)
     const V* part = static_cast<const V*>(A.part);
     const V* head = static_cast<const V*>(A.head);
     const V* tail = static_cast<const V*>(A.tail);
-    const uint32_t gb = (NORMLAP || A.mode == 2) ? 0u : *A.gbp;
+    const uint32_t gb = NORMLAP ? 0u : *A.gbp;
     const uint32_t nb = A.B.ncb > 1 ? A.B.ncb : 1u;
     double S[NS];
 #pragma unroll
@@ -1246,7 +1245,7 @@ __global__ void __launch_bounds__(BLOCK) k_power_finish(StepArgs A)
         if (A.ax) A.ax[r] = (double)v;  // the last one written is A u of the returned u
         const V xv = xform(yr, a, s);  // as the streaming kernel formed x
         const double xr = (double)xv;
-        const V yv = (V)shifted<NORMLAP>(A, (double)v, xr, wd, gb);
+        const V yv = (V)shifted<NORMLAP>((double)v, xr, wd, gb);
         yn[r] = yv;
         const double y = (double)yv;
         S[0] += NORMLAP ? 0.0 : y;
@@ -1271,7 +1270,7 @@ __global__ void __launch_bounds__(BLOCK) k_power_finish(StepArgs A)
                 for (int j = 0; j < 8; j++) v += h[j];
             }
             for (; q < nb; q++) v += part[q * A.n + r];
-            emit(r, yp[r], A.wdeg ? A.wdeg[r] : 0u, v);
+            emit(r, yp[r], A.wdeg[r], v);
         }
     }
     if (!MANY && nb == 1) {
@@ -1287,7 +1286,7 @@ __global__ void __launch_bounds__(BLOCK) k_power_finish(StepArgs A)
                 s0[k] = A.rowptr[q];
                 s1[k] = A.rowptr[q + 1];
                 yr[k] = yp[q];
-                wd[k] = A.wdeg ? A.wdeg[q] : 0u;
+                wd[k] = A.wdeg[q];
             }
             uint32_t w0[RB], w1[RB];
 #pragma unroll
@@ -1320,7 +1319,7 @@ __global__ void __launch_bounds__(BLOCK) k_power_finish(StepArgs A)
         }
     }
     for (; r < A.n; r += stride)
-        emit(r, yp[r], A.wdeg ? A.wdeg[r] : 0u, row_total<KB, MANY>(A, r, nb, part, head, tail));
+        emit(r, yp[r], A.wdeg[r], row_total<KB, MANY>(A, r, nb, part, head, tail));
     if (A.mode != 0) return;
     double tot[NS];
     block_sum_k<NS>(S, tot, red);
@@ -1424,7 +1423,7 @@ __global__ void __launch_bounds__(LBLOCK) k_power_small(StepArgs A, double* buf0
         for (uint32_t r = tid; r < A.n; r += LBLOCK) {
             const double v = row_total<1, false>(A, r, 1u, part, head, tail);
             const double xr = xl[r];
-            const double y = shifted<NORMLAP>(A, v, xr, A.wdeg ? A.wdeg[r] : 0u, gb);
+            const double y = shifted<NORMLAP>(v, xr, A.wdeg[r], gb);
             yn[r] = y;
             S[0] += NORMLAP ? 0.0 : y;
             S[1] += y * y;
@@ -1528,7 +1527,7 @@ __device__ __forceinline__ void small_loop(const StepArgs& A, double* buf0, doub
                 w0[k] = s0 >> A.B.pws;
                 w1[k] = (s1 - 1) >> A.B.pws;
             }
-            wd[k] = A.wdeg ? A.wdeg[r] : 0u;
+            wd[k] = A.wdeg[r];
         }
     }
     uint32_t iter = A.cnt[CT_ITER] + 1u;  // 1-based index of the next iteration
@@ -1621,7 +1620,7 @@ __device__ __forceinline__ void small_loop(const StepArgs& A, double* buf0, doub
                     for (uint32_t q = w0[k] + 1; q <= w1[k]; q++) v += hl[q];
                 }
                 const double xr = xl[r];
-                const double y = shifted<NORMLAP>(A, v, xr, wd[k], gb);
+                const double y = shifted<NORMLAP>(v, xr, wd[k], gb);
                 yl[r] = y;
                 S[0] += NORMLAP ? 0.0 : y;
                 S[1] += y * y;

@@ -63,25 +63,6 @@ __device__ __forceinline__ T ldc(const T* p)
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// largest of the lanes' values, in every lane
-__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v)
-{
-    // (a lane without a source keeps its own value)
-#define MI_STEP(CTRL, ROWS)                                                                             \
-    {                                                                                                   \
-        const uint32_t t = (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, ROWS, 0xf, false); \
-        v = t > v ? t : v;                                                                              \
-    }
-    MI_STEP(0x111, 0xf)  // row_shr:1, 2, 4, 8: lane 15 of each row of 16 holds the row's
-    MI_STEP(0x112, 0xf)
-    MI_STEP(0x114, 0xf)
-    MI_STEP(0x118, 0xf)
-    MI_STEP(0x142, 0xa)  // row_bcast:15, :31: lane 63 holds all
-    MI_STEP(0x143, 0xc)
-#undef MI_STEP
-    return (uint32_t)__builtin_amdgcn_readlane((int)v, WAVE - 1);
-}
-
 __device__ __forceinline__ long long wave_sum_i64(long long v)
 {
 #pragma unroll

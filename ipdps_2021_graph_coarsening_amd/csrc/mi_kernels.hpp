@@ -178,7 +178,7 @@ struct RowStep {
     void* ynew;
     double c, tol;
     unsigned long long iter_max;
-    int mode;                // 0: loop iteration, 1: one shifted product (a = 0, s = 1), 2: plain A x
+    int mode;                // 0: loop iteration, 1: one shifted product (a = 0, s = 1)
     uint32_t* cnt;
     int itr, itw;            // the counters of finished iterations that this launch reads and writes
     double* scal;

@@ -294,8 +294,8 @@ __device__ __forceinline__ uint32_t scalar_word(const uint32_t* p)
     return uniform(*(Const)(uintptr_t)p);
 }
 
-// One row: y from z = A y_prev (the shifted product of the reference, or A x
-// in mode 2), stored, and its terms of the sums.
+// One row: y from z = A y_prev (the shifted product of the reference), stored,
+// and its terms of the sums.
 template <class V>
 __device__ __forceinline__ void emit_row(const RowStep& A, uint32_t r, V z, V yr, uint32_t wd, uint32_t gb, double a,
                                          double s, double (&S)[sums_of<V>])
@@ -303,11 +303,7 @@ __device__ __forceinline__ void emit_row(const RowStep& A, uint32_t r, V z, V yr
     const double x = ((double)yr - a) * s;
     const double ax = s * ((double)z - a * (double)wd);
     if (A.ax) A.ax[r] = ax;  // the last one written is A u of the returned u
-    double y;
-    if (A.mode == 2)
-        y = ax;
-    else
-        y = fma((double)(uint32_t)(gb - wd), x, ax);
+    const double y = fma((double)(uint32_t)(gb - wd), x, ax);
     static_cast<V*>(A.ynew)[r] = (V)y;
     S[0] += y;
     S[1] = fma(y, y, S[1]);
@@ -344,14 +340,14 @@ __global__ void __launch_bounds__(BLOCK) k_power_rows(RowStep A)
     const uint32_t lane = threadIdx.x & (WAVE - 1), k = uniform(logical_block() * NW + threadIdx.x / WAVE);
     uint32_t sl = scalar_word(A.span + k);
     const uint32_t end = scalar_word(A.span + k + 1);
-    const uint32_t gb = A.mode == 2 ? 0u : *A.gbp;
+    const uint32_t gb = *A.gbp;
     V z = 0, yr = 0;
     uint32_t row = INF, wd = 0;
     auto slice = [&]() {
         row = A.row[(size_t)sl * WAVE + lane];
         const uint32_t g0 = scalar_word(A.soff + sl), g1 = scalar_word(A.soff + sl + 1);
         yr = row != INF ? yp[row] : (V)0;
-        wd = row != INF && A.wdeg ? A.wdeg[row] : 0u;
+        wd = row != INF ? A.wdeg[row] : 0u;
         z = 0;
         if (g0 < g1) {
             Group q, nx;

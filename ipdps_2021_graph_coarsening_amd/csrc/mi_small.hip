@@ -190,8 +190,6 @@ __device__ __forceinline__ double group_sum(double z, uint32_t t)
     return z;
 }
 
-__device__ __forceinline__ uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
-
 // Max / sum over the workgroup, in every thread.
 template <int NWV>
 __device__ __forceinline__ uint32_t max_all(uint32_t v, uint32_t* lds)
