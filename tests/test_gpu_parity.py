@@ -317,7 +317,7 @@ def test_power_iter_graph_replay_equals_eager(ctx, normLap):
     (each level captures its own graph; eager work runs between them)."""
     rng = np.random.default_rng(21 + normLap)
     cases = [random_graph(rng, 3000, 0.002, weighted=True, lcc=True), _hub_graph(3),
-             _dense_graph(20000, 70, 5, True)]
+             _dense_graph(20000, 70, 5, True), graphs.grid2d(120)]  # (the last: rows of at most 128 entries)
     try:
         for rp, col, w in cases:
             g = ctx.graph(rp, col, w)
@@ -576,24 +576,24 @@ def test_context_destroyed_before_its_objects():
 
 
 @pytest.mark.parametrize("normLap", [0, 1])
-@pytest.mark.parametrize("case", ["er3000w", "grid64", "rmat11w_hubs", "grid80", "grid100", "hub8192", "hub8000"])
+@pytest.mark.parametrize("case", ["er3000w", "grid64", "rmat11w_hubs", "grid80", "grid84", "grid100", "hub8192",
+                                  "hub8000"])
 def test_small_level_workgroup_vs_steps_and_oracle(ctx, case, normLap):
-    """The one-workgroup loop of small levels (vectors in LDS up to 8192
-    vertices, 4 or 8 rows per thread: grid80 takes the 8-row form, grid100
-    the form with vectors in global memory)
-    against the two-kernel step (same stop rule, sums added in another
+    """The one-workgroup loops of small levels against the launches per
+    iteration that run without them (same stop rule, sums added in another
     order, the start vector's too: the FP64 tolerances used against the
     oracle) and against the oracle; launches resumed every 7 iterations, and
-    every iteration, equal one launch bit for bit."""
+    every iteration, equal one launch bit for bit.  Plain: k_small_chain up to
+    7168 vertices (grid84: 7056) against k_power_rows or, with hubs, the two
+    launches, k_power_small_lds on hub8192; grid100 and hub8000 take the same
+    launches either way.  Normalised: k_power_small_lds (4 rows per thread, from
+    grid80 on 8) and, on grid100, k_power_small against the two launches.  That
+    two forms ran is seen from the vectors' last bits."""
     rng = np.random.default_rng(21)
     if case == "er3000w":
         rp, col, w = random_graph(rng, 3000, 0.002, weighted=True, lcc=True)
-    elif case == "grid64":
-        rp, col, w = graphs.grid2d(64)
-    elif case == "grid80":
-        rp, col, w = graphs.grid2d(80)
-    elif case == "grid100":
-        rp, col, w = graphs.grid2d(100)
+    elif case.startswith("grid"):
+        rp, col, w = graphs.grid2d(int(case[4:]))
     elif case.startswith("hub"):  # the most entries that a plain level past 7168 vertices has in that form, and more
         n, m = int(case[3:]), 36864 if case == "hub8192" else 36866
         us, vs = [np.arange(n - 1), np.zeros(129, np.int64)], [np.arange(1, n), np.arange(2, 131)]
@@ -619,6 +619,7 @@ def test_small_level_workgroup_vs_steps_and_oracle(ctx, case, normLap):
         ctx.set_small_levels()
     assert itc == its and np.array_equal(uc, us)
     assert it1 == its and np.array_equal(u1, us)
+    assert np.array_equal(us, um) == (normLap == 0 and case in ("grid100", "hub8000"))
     assert abs(its - itm) <= max(2, ITER_SLACK * itm) and not mrs
     assert abs(us @ um) / (np.linalg.norm(us) * np.linalg.norm(um)) >= EV_COS
     if normLap == 0:

@@ -3,11 +3,16 @@ slice, 4 entries per group, sorted windows of 2048 rows) at the sizes where
 it can go wrong: the edges of a slice and of a window, rows of no entries, of
 whole and ragged groups, of 128 entries (the longest taken) and 129 (which the
 streaming step takes), unit weights, weights at the edge of 16 bits and past
-it, and a loop that ends after its first iteration.
+it, and a loop that ends after its first iteration.  With normLap the same
+levels take the streaming step.
 
 Reference: numpy FP64 of the same formulas (eigensolve_kokkos.h:102-206).  A
 product with a row of k entries differs by at most (k + 3) eps times the sum
-of the absolute terms; for the loop's vectors see test_gpu_small.py (1e-11)."""
+of the absolute terms; for the loop's vectors see test_gpu_small.py (1e-11).  With
+normLap the runs' vectors differ by e = |u - u_host|, the constant's part too,
+and two dot products of unit vectors by at most 2 e on either side (the step's
+norm is at least 1/2): 8 e are allowed on their change, which must stay far
+below tol."""
 import numpy as np
 import pytest
 import scipy.sparse as sp
@@ -107,10 +112,11 @@ def test_loop(ctx, n, degrees, longest, wmax, tol, normLap):
         v = v / np.linalg.norm(v)
         dots.append(h @ v)
     d = u - h
+    slack = 8 * np.linalg.norm(d) if normLap else 1e-6 * tol
+    assert slack <= 0.1 * tol
     if normLap:  # (the constant vector: see test_gpu_small.py)
         span = np.stack([np.ones(n), h], axis=1)
         d = d - span @ np.linalg.lstsq(span, d, rcond=None)[0]
     assert np.linalg.norm(d) <= 1e-11
-    if not normLap:
-        assert abs(dots[-1] - dots[-2]) <= tol * (1 + 1e-6)
-        assert abs(dots[-2] - dots[-3]) > tol * (1 - 1e-6)
+    assert abs(dots[-1] - dots[-2]) <= tol + slack
+    assert abs(dots[-2] - dots[-3]) > tol - slack
