@@ -48,7 +48,8 @@ typedef struct {
     int refine_alg;       /* 0: Laplacian, 1: normalised Laplacian (normLap):
                              the loop takes the constant vector out once, so
                              where it stops depends on the last bits of the
-                             sums; their order is the same for every call */
+                             sums, whose order a level and the context's
+                             settings determine */
     int local_search_alg; /* 0 only (the reference returns before local search); FM refinement is
                              the context's mi_ctx_set_refinement, as it is a build flag there */
     int num_iter;         /* trials; the library runs one trial per call */

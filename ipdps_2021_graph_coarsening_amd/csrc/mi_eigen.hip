@@ -1338,8 +1338,8 @@ __global__ void __launch_bounds__(BLOCK) k_power_finish(StepArgs A)
 // depends on the order of every sum.  These forms and the two-kernel step fix
 // that order for normLap; the faster forms of mi_small.hip and mi_rows.hip add
 // in another and are for the plain Laplacian, where the constant is taken out
-// in every iteration (of 140 normalised bisections of meshes 39 changed with
-// the order, by up to 26 % of the cut, of 240 plain ones none).  Every
+// in every iteration (of 140 normalised bisections of meshes 46 changed with
+// the order, by up to 26 % of the cut, of 400 plain ones none).  Every
 // iteration is the two-kernel step above in one place: the stop test on the
 // previous iteration's sums, x = (y - a) s staged in LDS, the ranges of
 // entries streamed by the 16 wavefronts in turn (stream_range, LDS form,
@@ -2993,22 +2993,29 @@ static void solve_lds_levels(Ctx& c, std::vector<LdsLevel>& lv, int normLap, dou
         DBuf<double> b0, b1;
     };
     std::vector<Own> own(J);
-    // per job: 8 counters, 16 scalars, the iteration count (zero = a fresh loop)
-    DBuf<uint32_t> cnt(&c.pool, 8 * J);
-    DBuf<double> scal(&c.pool, 16 * J);
-    DBuf<unsigned long long> nit(&c.pool, J);
-    MI_HIP(hipMemsetAsync(cnt.get(), 0, 32 * J, c.stream));
-    MI_HIP(hipMemsetAsync(scal.get(), 0, 128 * J, c.stream));
-    MI_HIP(hipMemsetAsync(nit.get(), 0, 8 * J, c.stream));
+    // one table: the jobs, their scalars, and what their loops end with (zero: a fresh loop)
+    struct End {
+        unsigned long long niter;
+        uint32_t cnt[8];
+    };
+    const size_t o_scal = J * sizeof(SmallJob), o_end = o_scal + J * 16 * sizeof(double),
+                 bytes = o_end + J * sizeof(End);
+    static_assert(sizeof(SmallJob) % 8 == 0 && sizeof(End) % 8 == 0, "the table's parts are 8-byte aligned");
+    std::vector<uint64_t> table(bytes / 8, 0);
+    SmallJob* host = reinterpret_cast<SmallJob*>(table.data());
+    DBuf<uint64_t> dev(&c.pool, bytes / 8);
+    char* dp = reinterpret_cast<char*>(dev.get());
+    const SmallJob* dj = reinterpret_cast<const SmallJob*>(dp);
+    End* dend = reinterpret_cast<End*>(dp + o_end);
     // jobs of at most 4 rows per thread first (their kernel instance keeps
-    // its rows' metadata in fewer registers), then the others
+    // its rows' metadata in fewer registers; plain levels are larger), then the others
+    const auto four = [&](size_t j) { return normLap && lv[j].g->n <= 4u * LBLOCK; };
     std::vector<size_t> order;
     for (size_t j = 0; j < J; j++)
-        if (lv[j].g->n <= 4u * LBLOCK) order.push_back(j);
+        if (four(j)) order.push_back(j);
     const size_t J4 = order.size();
     for (size_t j = 0; j < J; j++)
-        if (lv[j].g->n > 4u * LBLOCK) order.push_back(j);
-    std::vector<SmallJob> host(J);
+        if (!four(j)) order.push_back(j);
     unsigned long long cap = 0;
     for (size_t k = 0; k < J; k++) {
         const size_t j = order[k];
@@ -3022,11 +3029,11 @@ static void solve_lds_levels(Ctx& c, std::vector<LdsLevel>& lv, int normLap, dou
         weighted_degree(c, g, o.plan, o.wdeg.get(), o.gb.get());
         o.b0 = DBuf<double>(&c.pool, g.n);
         o.b1 = DBuf<double>(&c.pool, g.n);
-        SmallJob& h = host[k];
+        SmallJob& h = *new (&host[k]) SmallJob;
         h.A = make_args(c, g, o.plan, o.wdeg.get(), o.gb.get(), o.b0.get(), o.b1.get(), tol, 0);
-        h.A.cnt = cnt.get() + 8 * k;
-        h.A.scal = scal.get() + 16 * k;
-        h.A.niter = nit.get() + k;
+        h.A.cnt = dend[k].cnt;
+        h.A.scal = reinterpret_cast<double*>(dp + o_scal) + 16 * k;
+        h.A.niter = &dend[k].niter;
         h.A.fprev = o.plan.fsum.get();
         h.A.fcur = o.plan.fsum.get();
         h.b0 = o.b0.get();
@@ -3036,17 +3043,12 @@ static void solve_lds_levels(Ctx& c, std::vector<LdsLevel>& lv, int normLap, dou
         h.out = lv[j].out;
         cap = std::max(cap, h.A.iter_max);
     }
-    DBuf<uint64_t> jobs(&c.pool, (J * sizeof(SmallJob) + 7) / 8);
-    MI_HIP(hipMemcpyAsync(jobs.get(), host.data(), J * sizeof(SmallJob), hipMemcpyHostToDevice, c.stream));
-    const SmallJob* dj = reinterpret_cast<const SmallJob*>(jobs.get());
-    std::vector<uint32_t> hc(8 * J);
+    MI_HIP(hipMemcpyAsync(dp, table.data(), bytes, hipMemcpyHostToDevice, c.stream));
+    std::vector<End> end(J);
     for (unsigned long long launched = 0;; launched += c.small_chunk) {
         MI_CHECK(launched <= cap + c.small_chunk, ST_INTERNAL, "power iteration did not stop at its iteration cap");
         if (J4) {
-            if (normLap)
-                k_power_small_lds<true, 4><<<(unsigned)J4, LBLOCK, 0, c.stream>>>(dj, c.small_chunk);
-            else
-                k_power_small_lds<false, 4><<<(unsigned)J4, LBLOCK, 0, c.stream>>>(dj, c.small_chunk);
+            k_power_small_lds<true, 4><<<(unsigned)J4, LBLOCK, 0, c.stream>>>(dj, c.small_chunk);
             MI_HIP(hipGetLastError());
         }
         if (J > J4) {
@@ -3056,18 +3058,19 @@ static void solve_lds_levels(Ctx& c, std::vector<LdsLevel>& lv, int normLap, dou
                 k_power_small_lds<false, 8><<<(unsigned)(J - J4), LBLOCK, 0, c.stream>>>(dj + J4, c.small_chunk);
             MI_HIP(hipGetLastError());
         }
-        MI_HIP(hipMemcpyAsync(hc.data(), cnt.get(), 32 * J, hipMemcpyDeviceToHost, c.stream));
-        MI_HIP(hipStreamSynchronize(c.stream));
+        if (J == 1) {
+            read_words(c, dend, end.data(), sizeof(End));
+        } else {
+            MI_HIP(hipMemcpyAsync(end.data(), dend, J * sizeof(End), hipMemcpyDeviceToHost, c.stream));
+            MI_HIP(hipStreamSynchronize(c.stream));
+        }
         bool all = true;
-        for (size_t j = 0; j < J && all; j++) all = hc[8 * j + CT_DONE] != 0;
+        for (size_t k = 0; k < J && all; k++) all = end[k].cnt[CT_DONE] != 0;
         if (all) break;
     }
-    std::vector<unsigned long long> hn(J);
-    MI_HIP(hipMemcpyAsync(hn.data(), nit.get(), 8 * J, hipMemcpyDeviceToHost, c.stream));
-    MI_HIP(hipStreamSynchronize(c.stream));
     for (size_t k = 0; k < J; k++) {
-        lv[order[k]].iters = hn[k];
-        lv[order[k]].max_reached = hc[8 * k + CT_MAXR] ? 1 : 0;
+        lv[order[k]].iters = end[k].niter;
+        lv[order[k]].max_reached = end[k].cnt[CT_MAXR] ? 1 : 0;
     }
 }
 

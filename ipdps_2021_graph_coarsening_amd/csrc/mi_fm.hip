@@ -373,8 +373,8 @@ __device__ __forceinline__ uint32_t rdl(uint32_t v, int l) { return (uint32_t)__
 // neighbours of each other is found in registers (each lane compares its
 // previous / next vertex with the other lanes' vertices), so a run of
 // adjacent leaving vertices is walked lane to lane, and the stores of the
-// removals and insertions of one step go to distinct words.  Every step
-// begins by waiting for the previous step's stores.
+// removals and insertions of one step go to distinct words.  Only the form with
+// everything in device memory waits for a step's stores before the next.
 template <int AT>
 __global__ void __launch_bounds__(FM_BLOCK) k_fm_search(FmSearch a)
 {

@@ -437,7 +437,7 @@ __global__ void k_map_assign2(uint32_t n, const uint32_t* __restrict__ pos, cons
 // whatever its size (the maps of all levels of the 2d grid 64^2 0.29 ms by
 // launches and 0.12 ms so, of the random geometric graph of 100,003 vertices,
 // whose three largest are above the line, 0.85 and 0.55 ms).
-// nonact: heavy-neighbour children not yet known to be passive.
+// kids: heavy-neighbour children not yet known to be passive.
 // out: ids of pass 1, of pass 2, vertices left unresolved, the largest id.
 constexpr uint32_t MAP_LDS = 4096;
 constexpr int MAP_BLOCK = 1024;

@@ -11,11 +11,12 @@
 //
 // Layout: 64 rows, one per lane, are a slice; the entries of a slice lie group
 // by group, GROUP consecutive entries of each lane's row in one 16-byte load
-// of columns.  Rows are taken in windows of WIN, sorted by their number of
-// groups, so that the rows of a slice have about the same number and padding
-// stays small, while the vector values they touch stay within the window's
-// lines.  Padding entries have weight 0 and the column n, where the vectors
-// hold a zero.
+// of columns (sliced ELLPACK with sorting windows: SELL-C-sigma, Kreutzer et
+// al., SIAM J. Sci. Comput. 36, 2014).  Rows are taken in windows of WIN, sorted
+// by their number of groups, so that the rows of a slice have about the same
+// number and padding stays small, while the vector values they touch stay
+// within the window's lines.  Padding entries have weight 0 and the column n,
+// where the vectors hold a zero.
 //
 // The deflation and normalisation of an iteration are never written back (as
 // in the streaming step): the next one reads its input as x = (y - a) s.  Here
@@ -325,7 +326,8 @@ __device__ __forceinline__ void leave_sums(const RowStep& A, const double (&S)[N
 }
 
 // Bound by memory on large levels and by the chain counter, sums, entries,
-// gathers on small ones (one launch is not shorter than about 7 us).  us per
+// gathers on small ones (the kernel of a level of 8,000 to 20,000 vertices
+// takes 4.5 to 6 us, an iteration with its launch 6.5 at least).  us per
 // iteration, the streaming step's two launches before and this one: 3d grid
 // 128^3 in FP64 73 and 47 (2.2 TB/s of the layout and vectors; the gathers of
 // neighbours a plane away miss L1), its level of 628,115 vertices 44 and 35,
@@ -403,8 +405,11 @@ void launch(Ctx& c, const RowStep& A)
 bool plan_rows(Ctx& c, const DGraph& g, RowPlan& p)
 {
     const uint32_t n = g.n, m = g.m;
-    // (levels of longer rows on average nearly always hold some past
-    // SHORT_ROW: they are not searched for one)
+    // (power-law levels of longer rows on average hold some past SHORT_ROW: they
+    // are not searched for one, some 15 us.  Regular stencils of 33 to 128
+    // entries a row stay with the streaming step that way, though this one is
+    // faster on them: 49,729 vertices, 40 entries a row 12.6 us per iteration and
+    // 7.1, 60 a row 18.7 and 8.4; 199,809, 60 a row 40 and 19.)
     if (!m || (uint64_t)m > (uint64_t)(SHORT_ROW / 4) * n) return false;
     const uint32_t ncu = c.num_cu > 0 ? (uint32_t)c.num_cu : 256u;
     // longest row, and (at once where that is little to read) largest weight

@@ -879,9 +879,15 @@ __global__ void __launch_bounds__(NWV * WAVE, NWV / 4)
     }
 }
 
-// Matrix words of a level outside LDS at most: every class of rows pads its
-// first slice to at most its longest row, and each slice to whole steps
-// (together below m + n + 16384 words); wide entries take two words.
+// Matrix words of a level outside LDS at most.  A slice is padded to its
+// longest row; rows are sorted, so all of a class but the first slice hold at
+// most the entries of the slice before.  That first one has 64 lanes of at most
+// 28 steps (one T for every row: 128), or rows of 64 lanes, which need no
+// padding among each other.  Rounding rows up to whole steps or groups adds at
+// most m / 3 (rows of T lanes have more than 3 T entries, in whole groups more
+// than 12 T) and, for the rows of the smallest T, 4 n or 2,048; the last group of
+// each wavefront 3 steps.  Together below 4/3 m + 4 n + 16384 words; wide
+// entries take two.
 uint64_t matrix_words(const DGraph& g)
 {
     const uint64_t words = 2ull * g.m + 8ull * g.n + 16384;
