@@ -49,7 +49,9 @@ constexpr int W_UNIT = 0, W_U16 = 1, W_U32 = 2;  // weight formats
 
 inline unsigned grid1(uint64_t n) { return (unsigned)ceil_div(n ? n : 1, BLOCK); }
 
-// longest row and largest weight: out[0], out[1] (zeroed before)
+// longest row and largest weight: out[0], out[1] (zeroed before).  A workgroup
+// that meets a row past SHORT_ROW, which decides the matter, leaves the weights
+// (a product with its plan on R-MAT-20, edge factor 6: 0.81 ms, 0.76 ms so).
 __global__ void __launch_bounds__(BLOCK) k_extremes(uint32_t n, uint64_t m, const uint32_t* __restrict__ rowptr,
                                                     const uint32_t* __restrict__ w, uint32_t* __restrict__ out)
 {
@@ -60,9 +62,9 @@ __global__ void __launch_bounds__(BLOCK) k_extremes(uint32_t n, uint64_t m, cons
         const uint32_t d = rowptr[r + 1] - rowptr[r];
         len = d > len ? d : len;
     }
-    if (w)
-        for (uint64_t e = t; e < m; e += step) wm = w[e] > wm ? w[e] : wm;
     len = block_max_u32(len, lds);
+    if (w && len <= SHORT_ROW)
+        for (uint64_t e = t; e < m; e += step) wm = w[e] > wm ? w[e] : wm;
     wm = block_max_u32(wm, lds);
     if (threadIdx.x == 0) {
         if (len) atomicMax(&out[0], len);
@@ -327,7 +329,7 @@ __device__ __forceinline__ void leave_sums(const RowStep& A, const double (&S)[N
 
 // Bound by memory on large levels and by the chain counter, sums, entries,
 // gathers on small ones (the kernel of a level of 8,000 to 20,000 vertices
-// takes 4.5 to 6 us, an iteration with its launch 6.5 at least).  us per
+// takes 4 to 6 us, an iteration with its launch 6.5 at least).  us per
 // iteration, the streaming step's two launches before and this one: 3d grid
 // 128^3 in FP64 73 and 47 (2.2 TB/s of the layout and vectors; the gathers of
 // neighbours a plane away miss L1), its level of 628,115 vertices 44 and 35,
