@@ -724,10 +724,10 @@ __device__ __forceinline__ void iterate_stream(const SmallLevel& V, const Layout
 // waits for a launch that finds that one done.
 // A level that the registers of eight wavefronts do not hold (rows of hundreds
 // of entries whose padding does not fit, or weights past 16 bits) is left to
-// sixteen, launched in the next round: eight hide its loads worse when they
-// stream it (R-MAT level of 388 vertices and 49,268 entries 15.6 us per
-// iteration against 10.0; 400 and 37,654 with heavy weights 11.4 against 7.6;
-// 200 and 15,374 4.6 against 3.4).
+// sixteen, which the host launches when it sees that: eight hide its loads
+// worse when they stream it (R-MAT level of 388 vertices and 49,268 entries
+// 15.6 us per iteration against 10.0; 400 and 37,654 with heavy weights 11.4
+// against 7.6; 200 and 15,374 4.6 against 3.4).
 template <int NWV>
 __global__ void __launch_bounds__(NWV * WAVE, NWV / 4)
     k_small_chain(const SmallJob* __restrict__ jobs, uint32_t chunk, double tol)

@@ -25,6 +25,7 @@ import numpy as np
 import pytest
 import scipy.sparse as sp
 
+import ipdps_2021_graph_coarsening_amd as mi
 from ipdps_2021_graph_coarsening_amd import graphs
 
 pytestmark = pytest.mark.gpu
@@ -179,6 +180,48 @@ def test_level_passed_on_to_sixteen_wavefronts(ctx, sizes, wmax):
     hu, dots = _host(rp, col, w, u0, 0, runs[0][1])
     assert np.linalg.norm(runs[0][0] - hu) <= 1e-11
     assert abs(dots[-1] - dots[-2]) <= TOL * (1 + 1e-6)
+
+
+def test_level_passed_on_inside_a_chain(ctx):
+    """A finest level whose weights fit 16 bits, coarser ones whose sums do not:
+    eight wavefronts leave those to sixteen and take the finest again.  Whole
+    chains in launches of 1, 50 and 8192 iterations, alone and in a batch with
+    a chain that needs no sixteen, give the same bits; against the launches
+    per iteration the vectors agree to 1e-6 (the same stop, other sums)."""
+    rp, col, _ = graphs.grid2d(75)
+    rng = np.random.default_rng(4)
+    r = np.repeat(np.arange(len(rp) - 1), np.diff(rp))
+    w = rng.integers(20000, 60001, len(col)).astype(np.uint32)
+    key = np.minimum(r, col).astype(np.int64) * len(rp) + np.maximum(r, col)
+    w = w[np.unique(key, return_index=True)[1]][np.searchsorted(np.unique(key), key)]  # symmetric
+    g, plain = ctx.graph(rp, col, w), ctx.graph(*graphs.grid2d(60))
+    H = g.hierarchy(5)
+    a = [H.level(l) for l in range(H.nlevels)]
+    eight = [l for l in range(H.nlevels)
+             if (a[l]["rowptr"][-1] > 5120 or len(a[l]["rowptr"]) > 1025)]
+    assert len(eight) >= 2 and a[0]["w"].max() <= 65535 and all(a[l]["w"].max() > 65535 for l in eight[1:])
+    cfg = mi.Config(4, 0, 0, 1, 1e-10, 2)
+    sols, parts = [], []
+    try:
+        for chunk in (0, 50, 1):
+            ctx.set_small_levels(1 << 17, chunk)
+            ev, st, _ = H.fiedler(9)
+            sols.append((ev, st["level_iters"]))
+            res, _ = mi.bisect_batch(ctx, [plain, g, plain], cfg, hec_seeds=[5] * 3, pcg_states=[9] * 3)
+            parts.append([x.part for x in res])
+        one = mi.partition_graph(ctx, g, cfg, hec_seed=5, pcg_state=9).part
+        ctx.set_small_levels(0)
+        ev, _, _ = H.fiedler(9)
+    finally:
+        ctx.set_small_levels()
+        H.close()
+        g.close()
+        plain.close()
+    for k in (1, 2):
+        assert sols[k][1] == sols[0][1] and np.array_equal(sols[k][0], sols[0][0])
+        assert all(np.array_equal(x, y) for x, y in zip(parts[k], parts[0]))
+    assert np.array_equal(parts[0][1], one) and np.array_equal(parts[0][0], parts[0][2])
+    assert abs(ev @ sols[0][0]) >= (1 - 1e-6) * np.linalg.norm(ev) * np.linalg.norm(sols[0][0])
 
 
 def test_rows_without_entries(ctx):
